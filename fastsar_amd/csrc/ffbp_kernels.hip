@@ -1364,6 +1364,12 @@ int launch_final_tiles(const float2* data, int B, int Pf, int Qf, int T, const d
     if (B < 1 || Pf < 1 || Qf < 1) { set_error("final_tiles: invalid shape"); return E_INVALID; }
     const char* force = getenv("FSH_FINAL_KERNEL");
     if (!(force && strcmp(force, "lds") == 0)) {
+        // T 16 and 32 at 8 lanes a block or more (fewer than 16,384 8 x 8 pixel blocks): on the matrix instructions,
+        // which sum a pixel's terms in another order; larger images keep one lane's order over (p, q) (a bright
+        // pixel's rounding stands out against the image's rms by the square root of its pixels)
+        if (T >= 16 && split >= 8)
+            return launch_final_tiles_mfma(data, B, Pf, Qf, T, ux, uy, tgeo, spx, spy, a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy,
+                                           nx, ny, out, s, split);
         const int per = (T / std::min(T, 8)) * (T / std::min(T, 8));
         const long blocks = ((long)B * per * split + 255) / 256;
         const bool w = w0 != nullptr;

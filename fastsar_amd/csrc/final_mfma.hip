@@ -1,0 +1,185 @@
+// The final stage of 16 x 16 and 32 x 32 tiles of images with few tiles, on the float32 matrix instructions: per tile
+//   out[i, j] = sum_{p, q} A[i; p, q] B[p, q; j],   A = d[p, q] exp(-2 pi i ux_p dlx_i (a0 + a1 q)) (w0 + gx dlx_i),
+//                                                 B =         exp(-2 pi i uy_p dly_j (a0 + a1 q)) (1 + gyr dly_j),
+// then the quadratic phase of each pixel and the cropped write (fastsar/ffbp_cpu.cpp:302-469).
+//
+// A workgroup forms an FB x FB block of a tile (FB 16, or 32 where there are tiles enough), each wave taking PC = 256 /
+// FB subapertures at a time and walking their samples q. A lane builds one run of 8 table entries (rows 8 c .. 8 c + 7
+// of A or B) of one subaperture: the run's first entry and its ratio seeded in float64 at q = 0 and advanced over q by
+// their own ratios, the entries by repeated products with the ratio (k_final_tiles_reg's tables, bit for bit). The
+// entries go through the wave's own LDS into the operand layout of v_mfma_f32_16x16x4_f32 (lane l: row or column l % 16,
+// contraction index l / 16, here the subaperture), four products a 16 x 16 block (Re Re, Im Im, Re Im, Im Re) into
+// independent accumulators. Waves' sums meet in LDS at the end, in wave order; images do not depend on the launch's
+// tile range.
+//
+// The float32 matrix instructions do the VALU's float32 rate (154 TFLOP/s) and take turns with its instructions. What
+// they change is that a pixel block no longer lives in one lane's registers: 64 lanes share 256 or 1,024 pixels' tables
+// and sums, so that an image of few tiles runs four or more waves a SIMD where one 8 x 8 block a lane ran a quarter to
+// one wave (final stage of 64 tiles of 32 x 32 with 103 x 72 samples 351 -> 60 us, of 768 with 102 x 91 994 -> 560 us,
+// of 576 of 16 x 16 with 113 x 64 and weights 512 -> 140 us). Bound by the two pipes' sum: 512 matrix cycles a step of
+// PC samples (1,024 at FB 32) and about 240 for the tables and their passage.
+#include "fsh_common.h"
+#include "fsh_kernels.h"
+
+#include <algorithm>
+
+namespace fsh {
+
+namespace {
+
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+constexpr int FW_MAX = 8;                  // waves a workgroup
+
+template <int FB>
+struct FinalShape {
+    static constexpr int PC = 256 / FB;            // subapertures a wave takes at a time
+    static constexpr int RS = PC + (FB == 16 ? 2 : 1);    // row stride of the tables (float2), spread over the banks
+    static constexpr int ESZ = 2 * FB * RS;        // table entries (float2) a wave
+};
+
+}  // namespace
+
+template <int T, int FB, bool W>
+__global__ __launch_bounds__(64 * FW_MAX) void k_final_tiles_mfma(const float2* __restrict__ data, int Pf, int Qf,
+                                                                  const double* __restrict__ ux, const double* __restrict__ uy,
+                                                                  const double* __restrict__ tgeo, double spx, double spy,
+                                                                  double a0, double a1, double fc2, const float* __restrict__ w0,
+                                                                  const float* __restrict__ gx, const float* __restrict__ gyr,
+                                                                  const int* __restrict__ tile_xy, int ox, int oy, int nx, int ny,
+                                                                  float2* __restrict__ out)
+{
+    typedef FinalShape<FB> S;
+    constexpr int PC = S::PC, RS = S::RS, NB = FB / 16, NS = T / FB;
+    extern __shared__ float2 lds[];                          // tables [waves][2 FB][RS], then sums [waves][FB][FB]
+    const int nw = blockDim.x >> 6;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // blocks are dispatched round-robin over the 8 XCDs: renumbered so that the blocks of one tile share an XCD's L2
+    int wg = blockIdx.x;
+    {
+        const int G = gridDim.x, q = G >> 3, rem = G & 7, xcd = wg & 7;
+        wg = xcd * q + min(xcd, rem) + (wg >> 3);
+    }
+    const int b = wg / (NS * NS), blk = wg - b * (NS * NS), bx = blk / NS, by = blk - bx * NS;
+    const double hc = 0.5 * (T - 1);
+    // table role: subaperture pl of the wave's PC, run ch; runs 0 .. FB / 8 - 1 are A's rows, the rest B's columns
+    const int pl = lane % PC, ch = lane / PC;
+    const bool isA = ch < FB / 8;
+    const int e0 = isA ? FB * bx + 8 * ch : FB * by + 8 * (ch - FB / 8);      // the run's first row or column of the tile
+    const double sp = isA ? spx : spy, dl0 = (e0 - hc) * sp;
+    float2* E = lds + wv * S::ESZ;
+    float2* ew = E + 8 * ch * RS + pl;
+    // product role: row or column i, contraction index k
+    const int i = lane & 15, k = lane >> 4;
+    const float2* ea = E + i * RS + k;
+    const float2* eb = ea + FB * RS;
+    floatx4_t rr[NB][NB], ii[NB][NB], ri[NB][NB], ir[NB][NB];
+    #pragma unroll
+    for (int m = 0; m < NB; ++m)
+        #pragma unroll
+        for (int n = 0; n < NB; ++n) rr[m][n] = ii[m][n] = ri[m][n] = ir[m][n] = floatx4_t{};
+
+    for (int p0 = PC * wv; p0 < Pf; p0 += PC * nw) {
+        const bool pok = p0 + pl < Pf;
+        const size_t bp = (size_t)b * Pf + min(p0 + pl, Pf - 1);
+        const float2* dq = data + bp * Qf;
+        float2 dn = load_ahead(dq);                    // the next sample, read one ahead
+        const double g = (isA ? ux : uy)[bp];
+        float2 r, sr, ba, sb;
+        cis_cyc(-(g * sp) * a0, r.x, r.y);             // ratio along the run at q = 0
+        cis_cyc(-(g * sp) * a1, sr.x, sr.y);           // its step over q
+        cis_cyc(-(g * dl0) * a0, ba.x, ba.y);          // the run's first entry, q = 0
+        cis_cyc(-(g * dl0) * a1, sb.x, sb.y);
+        float wt[8];
+        if (W) {
+            const float c0 = isA ? w0[bp] : 1.f, c1 = (isA ? gx : gyr)[bp];
+            #pragma unroll
+            for (int e = 0; e < 8; ++e) wt[e] = c0 + c1 * (float)(dl0 + e * sp);
+        }
+        const int steps = min(PC, Pf - p0 + 3) >> 2;   // contraction steps of four subapertures that hold one
+        for (int q = 0; q < Qf; ++q) {
+            // B's lanes take 1 in the sample's place, subapertures past the last 0
+            float2 v = cmul(isA ? (pok ? dn : make_float2(0.f, 0.f)) : make_float2(1.f, 0.f), ba);
+            dn = load_ahead(dq + min(q + 1, Qf - 1));
+            #pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                ew[e * RS] = W ? make_float2(v.x * wt[e], v.y * wt[e]) : v;
+                if (e < 7) v = cmul(v, r);
+            }
+            r = cmul(r, sr);
+            ba = cmul(ba, sb);
+            wave_lds_sync();
+            #pragma unroll
+            for (int s = 0; s < PC / 4; ++s) {
+                if (s < steps) {
+                    float2 a[NB], c[NB];
+                    #pragma unroll
+                    for (int m = 0; m < NB; ++m) { a[m] = ea[16 * m * RS + 4 * s]; c[m] = eb[16 * m * RS + 4 * s]; }
+                    #pragma unroll
+                    for (int m = 0; m < NB; ++m)
+                        #pragma unroll
+                        for (int n = 0; n < NB; ++n) {
+                            rr[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m].x, c[n].x, rr[m][n], 0, 0, 0);
+                            ii[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m].y, c[n].y, ii[m][n], 0, 0, 0);
+                            ri[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m].x, c[n].y, ri[m][n], 0, 0, 0);
+                            ir[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m].y, c[n].x, ir[m][n], 0, 0, 0);
+                        }
+                }
+            }
+            wave_lds_sync();
+        }
+    }
+    __syncthreads();                                   // every wave is done with its tables
+    // result element r of a lane: row 4 k + r, column i of its 16 x 16 block
+    #pragma unroll
+    for (int m = 0; m < NB; ++m)
+        #pragma unroll
+        for (int n = 0; n < NB; ++n)
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                lds[(wv * FB + 16 * m + 4 * k + r) * FB + 16 * n + i] =
+                    make_float2(rr[m][n][r] - ii[m][n][r], ri[m][n][r] + ir[m][n][r]);
+    __syncthreads();
+    const double cx = tgeo[3 * b], cy = tgeo[3 * b + 1], f = fc2 / (2.0 * tgeo[3 * b + 2]);
+    const int X0 = tile_xy[2 * b] - ox, Y0 = tile_xy[2 * b + 1] - oy;
+    for (int t = tid; t < FB * FB; t += blockDim.x) {
+        float2 v = lds[t];
+        for (int w = 1; w < nw; ++w) {
+            const float2 u = lds[w * FB * FB + t];
+            v.x += u.x;
+            v.y += u.y;
+        }
+        const int pi = FB * bx + t / FB, pj = FB * by + t % FB, X = X0 + pi, Y = Y0 + pj;
+        if (X < 0 || X >= nx || Y < 0 || Y >= ny) continue;
+        const double dx = (pi - hc) * spx, dy = (pj - hc) * spy;
+        const double los = cx * dx + cy * dy;
+        float cs, sn;
+        cis_cyc((dx * dx + dy * dy - los * los) * f, cs, sn);
+        out[(size_t)X * ny + Y] = cmul(v, make_float2(cs, sn));
+    }
+}
+
+int launch_final_tiles_mfma(const float2* data, int B, int Pf, int Qf, int T, const double* ux, const double* uy,
+                            const double* tgeo, double spx, double spy, double a0, double a1, double fc2, const float* w0,
+                            const float* gx, const float* gyr, const int* tile_xy, int ox, int oy, int nx, int ny, float2* out,
+                            hipStream_t s, int split)
+{
+    // split 8: an image of 256 to 512 tiles of 32 x 32 or more, whose 32 x 32 blocks fill the device; 16: fewer
+    const int FB = T == 32 && split < 16 ? 32 : 16, PC = FinalShape<16>::PC;
+    // four waves, a SIMD each (5 or 7 leave the SIMDs uneven: the 768 tiles above took 712 and 642 us); eight of 16 x 16
+    // blocks with the runs to share
+    const int nw = FB == 16 && Pf > 4 * PC ? FW_MAX : 4;
+    const long G = (long)B * (T / FB) * (T / FB);
+    if (G > 2147483647L) { set_error("final_tiles: too many tiles"); return E_INVALID; }
+    const dim3 grid((unsigned)G), block(64 * nw);
+    const size_t lds = nw * sizeof(float2) * std::max<size_t>(FB == 32 ? FinalShape<32>::ESZ : FinalShape<16>::ESZ, FB * FB);
+#define FSH_FM(TT, BB, WW) hipLaunchKernelGGL((k_final_tiles_mfma<TT, BB, WW>), grid, block, lds, s, data, Pf, Qf, ux, uy, tgeo, \
+                                              spx, spy, a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy, nx, ny, out)
+    if (T == 16) { if (w0) FSH_FM(16, 16, true); else FSH_FM(16, 16, false); }
+    else if (FB == 16) { if (w0) FSH_FM(32, 16, true); else FSH_FM(32, 16, false); }
+    else { if (w0) FSH_FM(32, 32, true); else FSH_FM(32, 32, false); }
+#undef FSH_FM
+    FSH_TRY(hipGetLastError());
+    return OK;
+}
+
+}  // namespace fsh
