@@ -1198,6 +1198,19 @@ bool fir_p_streams(int L, int D)
     return D >= 1 && (L + D - 1) / D <= 16 && !force;
 }
 
+// output pulses per segment of the streaming kernels (a thread runs down a column's rows of one segment, and the
+// segments of a column re-read ceil(L / D) - 1 periods of rows, from cache): at most 128, fewer where the columns alone
+// leave the launch short of 1,280 blocks (five a CU), not below 8. Measured, 128 against the rule: 64 x 157 columns of
+// 512 rows (62 MB) 141 -> 33 us, 48 x 301 of 1,403 186 -> 59, 64 x 264 of 3,000 380 -> 172, 64 x 352 of 4,096 425 -> 285;
+// 56 x 523 of 8,190 takes 128 either way (691 us; 745 at 24)
+static int fir_p_segment(long columns, int Po)
+{
+    if (const char* e = getenv("FSH_FIRP_IC")) return std::min(Po, std::max(1, atoi(e)));          // sweeps
+    const long per = (columns + 255) / 256;
+    const int segs = (int)((1280 + per - 1) / per);
+    return std::min(Po, std::min(128, std::max(8, (Po + segs - 1) / segs)));
+}
+
 int launch_fir_p(const float2* y, int B, int P, int Ko, const float* taps, int L, int pl, int D, int Po, float2* z, hipStream_t s,
                  const float* hs, const DeferredRot* rot, int ys, bool split)
 {
@@ -1219,9 +1232,7 @@ int launch_fir_p(const float2* y, int B, int P, int Ko, const float* taps, int L
     }
     const int sp = split ? 1 : 0;
     if (NW <= 16 && !(force && strcmp(force, "lds") == 0)) {
-        int IC = 128;                                                    // output pulses per segment
-        if (const char* e = getenv("FSH_FIRP_IC")) IC = std::max(1, atoi(e));          // sweeps
-        IC = std::min(Po, IC);
+        const int IC = fir_p_segment((long)B * Ko, Po);
         dim3 grid((unsigned)(((long)B * Ko + 255) / 256), (Po + IC - 1) / IC);
         const bool batch = force && strcmp(force, "stream4") == 0;
         const float* rc0 = rot ? rot->c0 : nullptr;
