@@ -468,14 +468,22 @@ bool level_mfma_shape(int Np, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int
     if (Dk * (16 * JT + NWp) > maxi * nthr || Dk * NWp > TAB_MAX || CB * NE > ef_items(tpw) * nthr ||
         CB * (4 * JT + 1) > (tpw == 1 ? 1 : 2) * nthr)
         return false;
-    // segments of output pulses: enough blocks to fill the device, a halo below a fifth of the rows
-    const long blocks0 = (long)Np * ((C + CB - 1) / CB) * njr;
-    nseg = 1;
-    long want = 2048;
-    if (const char* e = getenv("FSH_LMFMA_BLOCKS")) want = std::max(1, atoi(e));     // sweeps
-    while (nseg < Po && blocks0 * nseg < want && (long)Dp * ((Po + 2 * nseg - 1) / (2 * nseg)) >= 5L * Lp) nseg *= 2;
-    IS = (Po + nseg - 1) / nseg;
-    nseg = (Po + IS - 1) / IS;
+    // segments of output pulses, each re-reading Lp rows: the count with the least time by a model of the walk. A CU holds
+    // `occ` blocks (LDS, four waves a SIMD); k blocks on it take 1 + 0.06 (k - 1) nwv times one block's time a row (a
+    // barrier a row: measured 1.35-1.48 for two blocks of 6 or 7 waves, 1.43 from two to four of 4, 1.18 of 3), and a
+    // block's start about 12 rows' time. The halving rule before (2,048 blocks, a halo below a fifth) left images of few
+    // parents on a quarter of the CUs: 64 parents of 4 children, 266 rows 181 -> 100 us (8 segments for 1), 25 of 9, 477
+    // rows 355 -> 164, 16 of 4, 190 rows 125 -> 40; and cut past a whole round: 56 of 48, 2,058 rows 3.26 -> 3.02 ms
+    const int occ = std::max(1, std::min((int)(160 * 1024 / lds), 16 / nwv));
+    auto load = [&](long k) { return k ? 1.0 + 0.06 * (k - 1) * nwv : 0.0; };
+    double best = 0.0;
+    IS = 0;
+    for (int n = 1; n <= std::min(Po, 64); ++n) {
+        const int is = (Po + n - 1) / n, ns = (Po + is - 1) / is;
+        const long k = ((long)Np * ((C + CB - 1) / CB) * njr * ns + 255) / 256;
+        const double t = ((k / occ) * load(occ) + load(k % occ)) * ((double)Dp * is + Lp + 12);
+        if (!IS || t < best) { best = t; IS = is; nseg = ns; }
+    }
     return true;
 }
 
