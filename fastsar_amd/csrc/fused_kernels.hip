@@ -115,6 +115,18 @@ int launch_level_fused(const float2* x, int Np, int P, int K, const float* c0, c
     const int NWK = fused_nw(Lk, Dk), NWP = fused_nw(Lp, Dp);
     const long G = (long)Np * ((C + CB - 1) / CB);
     if (G > 2147483647L) { set_error("level_fused: too many parents"); return E_INVALID; }
+    // up to three blocks a CU: the CU's LDS shared among them, so that each walks its parent in fewer chunks (a chunk's
+    // range filter is one thread's walk along a row whatever the rows): 256 parents of 143 x 89 135 -> 86 us (64 rows a
+    // chunk for 15), 144 of 206 x 109 167 -> 127 (52 for 26), 576 of 211 x 96 298 -> 238 (19 for 29: one round of
+    // blocks, not two)
+    if (G <= 768 && !getenv("FSH_FUSED_LDS_KB")) {
+        const size_t per_row = 8 * ((size_t)(K | 1) + (size_t)CB * (Ko | 1)), kb = 156 / ((G + 255) / 256);
+        const int r = std::min(P, (int)std::min<size_t>(kb * 1024 / per_row, (size_t)(256 / CB)));
+        if (r >= 8 || r == P) {
+            R = r;
+            lds = per_row * R;
+        }
+    }
     const dim3 grid((unsigned)G), block(256);
     // the forms with both factors fixed where they cover the pair (FSH_FUSED_FIXED=0: the run-time form, for A/B)
     const char* fxe = getenv("FSH_FUSED_FIXED");
