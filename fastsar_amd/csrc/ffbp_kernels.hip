@@ -1163,6 +1163,11 @@ int launch_rot_fir_k(const float2* x, int Np, int P, int K, const float* c0, con
         if (st == E_INVALID) st = launch_rot_fir_k_mfma(x, Np, P, K, c0, sl, Cn, taps, L, pl, D, Ko, kc, y, s);
         if (st != E_INVALID) return st;
     }
+    // longer filters on the float32 matrix instructions where their window and taps fit LDS
+    if (!force && D > 1) {
+        const int st = launch_rot_fir_k_f32(x, Np, P, K, c0, sl, Cn, taps, L, pl, D, Ko, kc, y, s);
+        if (st != E_INVALID) return st;
+    }
     const int PB = 8;
     const int budget = std::min(lds_limit(), 65536);
     int JB = 64;

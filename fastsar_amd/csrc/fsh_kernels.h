@@ -29,6 +29,9 @@ inline int padded_row(int Ko) { return Ko >= 128 ? (Ko + 31) / 32 * 32 : Ko; }
 int launch_rot_fir_k_mf2(const float2* x, int Np, int P, int K, const float* c0, const float* sl, int Cn, const float* taps,
                          int L, int pl, int D, int Ko, double kc, float2* y, hipStream_t s, const float* hs = nullptr,
                          bool rot = true, int ys = 0);
+// the float32 matrix form for filters of more than 128 taps (range_f32.hip); E_INVALID when it does not fit LDS
+int launch_rot_fir_k_f32(const float2* x, int Np, int P, int K, const float* c0, const float* sl, int Cn, const float* taps,
+                         int L, int pl, int D, int Ko, double kc, float2* y, hipStream_t s);
 // the range stage's rho_b(p, j) = exp(2 pi i (c0[b P + p] + (D j - pl - kc) sl[b P + p])), left for the pulse filter
 struct DeferredRot {
     const float* c0;
