@@ -217,7 +217,13 @@ __device__ __forceinline__ void bp_region(const BpArgs& A)
     if (lg >= G) return;
     const int rx = A.along_e1 ? lg % A.nbx : lg / A.nby, ry = A.along_e1 ? lg / A.nbx : lg % A.nby;
     const int i0 = rx * BR, j0 = ry * BR;
-    const int tid = threadIdx.x, col = tid % BR, row = tid / BR;
+    // lanes run over 8 pixels along the across-range axis, then along the other: the pixels of one read lie at nearly 8
+    // ranges, whose bins (several apart from column to column) fall on different banks, and pixels at one range read the
+    // same words. With e1 across range and the lanes along e2 (32 ranges a read, two rows of them) the reads lost 47 % of
+    // their LDS cycles to conflicts, LDS busy 65 % of the time
+    const int tid = threadIdx.x;
+    const int col = A.along_e1 ? (tid >> 3) % BR : tid % BR;
+    const int row = A.along_e1 ? (tid & 7) + 8 * (tid / (8 * BR)) : tid / BR;
 
     // the pixels of this thread, all in one column: tile slot, integer row offset in the tile, metres from the tile
     // centre along e1, |d|^2; the column's offset and metres along e2 are the same for all of them
