@@ -173,6 +173,7 @@ __global__ __launch_bounds__(256) void k_to_half(const float2* __restrict__ win,
 struct BpArgs {
     const void* win;               // [n, W] cropped profiles of the chunk
     const unsigned* smax;          // float16 profiles: the chunk's largest magnitude
+    int seg;                       // pulses a block takes: block (region, s) pulses s seg .. (s + 1) seg - 1 into image s
     int P, W, nfft, NB, NWIN, TB;  // pulses of the chunk, window per pulse, FFT length, pulses per window batch,
                                    // LDS bins per window, pulses per batch of centre terms (a multiple of NB)
     const long long* blo;          // [n] first cropped bin of each pulse (zero delay at nfft / 2)
@@ -214,7 +215,9 @@ __device__ __forceinline__ void bp_region(const BpArgs& A)
     // forms at once then lie at nearly one range and read nearly the same window of each profile from its L2
     const int G = A.nbx * A.nby, per = (G + 7) / 8;
     const int lg = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (lg >= G) return;
+    const int pbeg = blockIdx.y * A.seg, pend = min(A.P, pbeg + A.seg);
+    if (lg >= G || pbeg >= pend) return;
+    float2* out = A.out + (size_t)blockIdx.y * A.nx * A.ny;
     const int rx = A.along_e1 ? lg % A.nbx : lg / A.nby, ry = A.along_e1 ? lg / A.nbx : lg % A.nby;
     const int i0 = rx * BR, j0 = ry * BR;
     // lanes run over 8 pixels along the across-range axis, then along the other: the pixels of one read lie at nearly 8
@@ -256,8 +259,8 @@ __device__ __forceinline__ void bp_region(const BpArgs& A)
     const float fdr = (float)A.inv_dr, fk = (float)A.kcyc;
     const float tmax = (float)(CUBIC ? NWIN - 3 : NWIN - 2) + 0.5f, tmin = CUBIC ? 1.f : 0.f;
 
-    for (int pt = 0; pt < A.P; pt += TB) {
-        const int ntb = min(TB, A.P - pt);
+    for (int pt = pbeg; pt < pend; pt += TB) {
+        const int ntb = min(TB, pend - pt);
         __syncthreads();                                   // the previous terms and windows are read
         // per pulse of the term batch, the first bin of the region's window
         for (int k = tid; k < ntb; k += 256) {
@@ -341,10 +344,10 @@ __device__ __forceinline__ void bp_region(const BpArgs& A)
         const int gi = i0 + row + RS * m, gj = j0 + col;
         if (gi < A.nx && gj < A.ny) {
             const size_t o = (size_t)gi * A.ny + gj;
-            float2 v = A.out[o];
+            float2 v = out[o];
             v.x = fmaf(ar[m], us, v.x);
             v.y = fmaf(ai[m], us, v.y);
-            A.out[o] = v;
+            out[o] = v;
         }
     }
 }
@@ -360,6 +363,20 @@ template <int BR, int TX, int TY, int PT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_bp_region_cubic(BpArgs A)
 {
     bp_region<BR, TX, TY, PT, true>(A);
+}
+
+// the sum of nseg images of n pixels, in order, into out (which may be the first of them)
+__global__ __launch_bounds__(256) void k_sum_images(const float2* im, size_t n, int nseg, float2* out)
+{
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        float2 v = im[i];
+        for (int k = 1; k < nseg; ++k) {
+            const float2 u = im[k * n + i];
+            v.x += u.x;
+            v.y += u.y;
+        }
+        out[i] = v;
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ float64 points
@@ -428,7 +445,8 @@ struct Exact {
     float* pinv = nullptr;           // a float16 history's per-pulse inverse scales (host input)
     double* ramp = nullptr;          // [P] (a, b) cycles: the phase re-reference applied on the way in (fsh_exact_set_ramp)
     bool use_ramp = false;
-    float2* image = nullptr;
+    float2* image = nullptr;         // [nseg, nx, ny]
+    int nseg = 1;                    // images the pulses of each chunk are dealt to (bp_segments)
     int* bad = nullptr;
     hipfftHandle plan = 0;
     int plan_n = 0;
@@ -503,11 +521,22 @@ static bool bp_shape(const fsh_exact_desc& d, BpShape& sh)
     return false;
 }
 
+// Images the pulses of a chunk are dealt to: a grid of few regions (1,024 pixels a workgroup, five workgroups a CU, each
+// one serial in its pulses) would leave the device idle, so that many workgroups share a region, up to 16, with 64
+// pulses or more each; their images are added at the end. From 641 regions up one image: two workgroups a region of
+// 1,024 regions would run in two rounds for one. 113 x 2,179 pixels (276 regions) from 1,916 pulses 2,400 -> 650 us, 121 x
+// 652 (84) from 628 1,398 -> 278, 1,568 x 261 (441) from 743 703 -> 474
+static int bp_segments(const fsh_exact_desc& d, int BR)
+{
+    const long G = (long)((d.nx + BR - 1) / BR) * ((d.ny + BR - 1) / BR);
+    return (int)std::max<long>(1, std::min<long>(std::min<long>(16, 1280 / G), std::min(d.chunk, d.P) / 64));
+}
+
 template <int BR, int TX, int TY, int PT>
 static void launch_region(const BpArgs& a, bool cubic, size_t lds, hipStream_t s)
 {
     const int G = a.nbx * a.nby;
-    const dim3 grid((unsigned)(8 * ((G + 7) / 8)));
+    const dim3 grid((unsigned)(8 * ((G + 7) / 8)), (unsigned)((a.P + a.seg - 1) / a.seg));
     if (cubic) hipLaunchKernelGGL((k_bp_region_cubic<BR, TX, TY, PT>), grid, dim3(256), lds, s, a);
     else hipLaunchKernelGGL((k_bp_region_linear<BR, TX, TY, PT>), grid, dim3(256), lds, s, a);
 }
@@ -540,6 +569,7 @@ static int launch_bp(const Exact& e, int n, int p0, float2* out)
     a.win = d.profiles ? e.winh : (const void*)e.win;
     a.smax = e.smax;
     a.P = n;
+    a.seg = e.nseg > 1 ? (std::min(d.chunk, d.P) + e.nseg * sh.NB - 1) / (e.nseg * sh.NB) * sh.NB : n;   // whole batches
     a.W = d.W;
     a.nfft = d.nfft;
     a.NB = sh.NB;
@@ -595,16 +625,15 @@ int fsh_exact_create(const fsh_exact_desc* desc, void** handle)
         set_error("exact_create: invalid descriptor");
         return E_INVALID;
     }
-    {
-        BpShape sh;
-        if (!bp_shape(d, sh)) {
-            set_error("exact_create: a pixel region's range window does not fit in LDS (use a smaller upsample or pixel "
-                      "spacing)");
-            return E_INVALID;
-        }
+    BpShape sh;
+    if (!bp_shape(d, sh)) {
+        set_error("exact_create: a pixel region's range window does not fit in LDS (use a smaller upsample or pixel "
+                  "spacing)");
+        return E_INVALID;
     }
     Exact* e = new Exact();
     e->d = d;
+    e->nseg = bp_segments(d, sh.BR);
     {
         // the line of sight from the track's mean to the grid's mean, against the grid's axes: the axis it has the
         // smaller part along is the across-range one
@@ -632,7 +661,7 @@ int fsh_exact_create(const fsh_exact_desc* desc, void** handle)
     if ((st = dev_alloc((void**)&e->pad, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->prof, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->win, (size_t)ch * d.W * sizeof(float2))) ||
-        (st = dev_alloc((void**)&e->image, (size_t)d.nx * d.ny * sizeof(float2))) || (st = dev_alloc((void**)&e->bad, sizeof(int))))
+        (st = dev_alloc((void**)&e->image, (size_t)e->nseg * d.nx * d.ny * sizeof(float2))) || (st = dev_alloc((void**)&e->bad, sizeof(int))))
         return fail(st);
     if (d.profiles && ((st = dev_alloc(&e->winh, (size_t)ch * d.W * (d.profiles == 2 ? 8 : 4))) ||
                        (st = dev_alloc((void**)&e->smax, sizeof(unsigned)))))
@@ -670,7 +699,7 @@ static int exact_form_impl(Exact* e, const void* S, int dtype, const float* puls
         if ((st = fft_status(hipfftSetStream(e->plan, e->stream), "hipfftSetStream"))) return st;
     }
     if ((st = launch_fill_int(e->bad, 1, INT_MAX, e->stream))) return st;
-    FSH_TRY(hipMemsetAsync(e->image, 0, (size_t)d.nx * d.ny * sizeof(float2), e->stream));
+    FSH_TRY(hipMemsetAsync(e->image, 0, (size_t)e->nseg * d.nx * d.ny * sizeof(float2), e->stream));
     for (int p0 = 0; p0 < d.P; p0 += ch) {
         const int n = std::min(ch, d.P - p0);
         if (n < ch) FSH_TRY(hipMemsetAsync(e->pad + (size_t)n * d.nfft, 0, (size_t)(ch - n) * d.nfft * sizeof(float2), e->stream));
@@ -710,6 +739,12 @@ static int exact_form_impl(Exact* e, const void* S, int dtype, const float* puls
             hipLaunchKernelGGL(k_to_half<true>, gw, dim3(256), 0, e->stream, e->win, n, d.W, e->smax, (half2_t*)e->winh);
         FSH_TRY(hipGetLastError());
         if ((st = launch_bp(*e, n, p0, e->image))) return st;
+    }
+    if (e->nseg > 1) {
+        const size_t n = (size_t)d.nx * d.ny;
+        hipLaunchKernelGGL(k_sum_images, dim3((unsigned)std::min<size_t>((n + 255) / 256, 1 << 16)), dim3(256), 0, e->stream,
+                           e->image, n, e->nseg, e->image);
+        FSH_TRY(hipGetLastError());
     }
     int badh = INT_MAX;
     FSH_TRY(hipMemcpyAsync(&badh, e->bad, sizeof(int), hipMemcpyDeviceToHost, e->stream));

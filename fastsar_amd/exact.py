@@ -287,9 +287,11 @@ class ExactFormer:
     def memory(self):
         """dict(backend, needed, available, full_speed, parts) in bytes. (fastsar/exact.py:736-761)"""
         ch = min(self.chunk, self.P)
+        # a grid of few 32 x 32 regions deals its pulses to up to 16 images (at most; fewer, larger windows take one)
+        images = max(1, min(16, 1280 // (-(-self.nx // 32) * -(-self.ny // 32)), ch // 64))
         parts = dict(history=self.P * self.K * 8, padded=ch * self.nfft * 8, fft=ch * self.nfft * 8,
                      window=ch * self.W * {'float32': 8, 'float16': 12, 'float16-pair': 16}[self.profiles],
-                     image=self.nx * self.ny * 8, geometry=self.cen.nbytes + self.P * 40)
+                     image=images * self.nx * self.ny * 8, geometry=self.cen.nbytes + self.P * 40)
         need = float(sum(parts.values()))
         avail = float(_hip.device_info()['mem'])
         return dict(backend=self.backend, needed=need, available=avail, full_speed=need <= avail, parts=parts)
