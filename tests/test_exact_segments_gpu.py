@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize('interp', ['cubic', 'linear'])
-@pytest.mark.parametrize('nx,ny,P', [(33, 31, 128), (7, 90, 129), (64, 65, 1024), (40, 100, 1100), (500, 250, 300)])
+@pytest.mark.parametrize('nx,ny,P', [(33, 31, 128), (7, 90, 129), (64, 65, 1024), (40, 100, 1100), (500, 200, 300)])
 def test_pulses_dealt_to_images(nx, ny, P, interp):
     rng = np.random.default_rng(P + nx)
     col = sim.spotlight(P, 256, 2.0)
