@@ -15,8 +15,12 @@
 //      cover it, a sliding window of accumulators; finished outputs go to an LDS block y [CB, R, Ko];
 //   3. one thread per (child, column j) streams the block's rows through the pulse filter the same way, its NWP
 //      accumulators persisting across chunks, and stores each finished output of z.
-// The sample loop's indices are the same for every lane, so the taps are read as uniform (scalar) loads from the
+// The sample loop's indices are the same for every lane, so the taps are uniform; they are read a chunk at a time from the
 // zero-padded polyphase tables hk_t[ph NWK + s] = hk[Dk (NWK - 1 - s) + ph] and hp_t likewise.
+//
+// Bound by VALU issue: of the 12288 x 8192 image's level 3 (2 x 3, 10 and 9 accumulators a filter) 38.0 ms with the taps in
+// scalar registers, 34.2 in vector registers (a scalar operand costs an fma 4.4 issue cycles for 2.5), 32.6 with the rows
+// padded by zeros (no clamp or check a sample), 31.8 with the pulse slots' shift folded into the period's first sums.
 #include "fsh_common.h"
 #include "fsh_kernels.h"
 #include "fused_level.h"
@@ -69,7 +73,7 @@ bool level_fused_shape(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int 
     if (Dk > DMAX || Dp > DMAX || fused_nw(Lk, Dk) < 0 || fused_nw(Lp, Dp) < 0 || Ko > 256 || C < 1 || P < 1 || K < 1)
         return false;
     CB = std::min(C, 256 / Ko);
-    const int KS = K | 1, KoS = Ko | 1;
+    const int KS = fused_row(K, Dk), KoS = Ko | 1;
     // 39 KB of rows a block: four blocks a CU (16 waves) hide the row loads' latency (the 12288 x 8192 image's level 3:
     // 53 ms against 69 ms at 78 KB, two blocks a CU); up to 78 KB where 39 KB would hold fewer than 16 rows
     size_t budget = 39 * 1024;
@@ -78,7 +82,11 @@ bool level_fused_shape(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int 
     R = (int)std::min<size_t>(budget / per_row, (size_t)(256 / CB));
     if (R < 16 && R < P && !getenv("FSH_FUSED_LDS_KB")) R = (int)std::min<size_t>(78 * 1024 / per_row, (size_t)(256 / CB));
     R = std::min(R, P);
-    if (R < 8 && R < P) return false;
+    if (R < 8 && R < P) {
+        // the rows' zeros do not turn a level away that fits without them
+        R = std::min(P, (int)std::min<size_t>(78 * 1024 / (8 * ((size_t)(K | 1) + (size_t)CB * KoS)), (size_t)(256 / CB)));
+        if (R < 8 && R < P) return false;
+    }
     lds = per_row * R;
     return true;
 }
@@ -120,7 +128,7 @@ int launch_level_fused(const float2* x, int Np, int P, int K, const float* c0, c
     // chunk for 15), 144 of 206 x 109 167 -> 127 (52 for 26), 576 of 211 x 96 298 -> 238 (19 for 29: one round of
     // blocks, not two)
     if (G <= 768 && !getenv("FSH_FUSED_LDS_KB")) {
-        const size_t per_row = 8 * ((size_t)(K | 1) + (size_t)CB * (Ko | 1)), kb = 156 / ((G + 255) / 256);
+        const size_t per_row = 8 * ((size_t)fused_row(K, Dk) + (size_t)CB * (Ko | 1)), kb = 156 / ((G + 255) / 256);
         const int r = std::min(P, (int)std::min<size_t>(kb * 1024 / per_row, (size_t)(256 / CB)));
         if (r >= 8 || r == P) {
             R = r;

@@ -9,6 +9,11 @@ namespace fsh {
 
 constexpr int DMAX = 4;                        // the largest decimation factor of the fused form, on either axis
 
+// Taps (uniform values) are moved to vector registers where a filter's fit VTAPS of them: a float32 fma whose operands
+// are all VGPRs issues in about 2.5 cycles a wave, one with a scalar operand in 4.4 (both at two or more waves a SIMD)
+constexpr int VTAPS = 32;
+__device__ __forceinline__ void in_vgpr(float& v) { asm volatile("" : "+v"(v)); }
+
 // f(std::integral_constant<int, I>) for I = B .. E - 1, unrolled at compile time
 template <int B, int E, typename F>
 __device__ __forceinline__ void static_for(F&& f)
@@ -18,6 +23,9 @@ __device__ __forceinline__ void static_for(F&& f)
         static_for<B + 1, E>(f);
     }
 }
+
+// the row stride of x in LDS (float2): the samples and Dk - 1 zeros on either side, odd
+__host__ __device__ inline int fused_row(int K, int Dk) { return (K + 2 * (Dk - 1)) | 1; }
 
 // DK, DP: the range and pulse decimation factors fixed at compile time (the loops over phases exact, half the taps
 // or fewer in scalar registers), or 0: read at run time, the loops running to DMAX with the phases past it skipped
@@ -39,11 +47,17 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
     }
     const int n = wg / nCB, cb = wg - n * nCB;
     const int cbeg = cb * CB, cn = min(CB, C - cbeg);
-    const int KS = K | 1, KoS = Ko | 1;
+    // a row of x in LDS: Dk - 1 zeros, its K samples, Dk - 1 zeros, so that a period partly outside [0, K) reads zeros and
+    // no read is checked or clamped
+    const int pad = (DK ? DK : Dk) - 1, KS = fused_row(K, DK ? DK : Dk), KoS = Ko | 1;
     float2* xs = lds_f2;                       // [R][KS]
     float2* ys = xs + (size_t)R * KS;          // [cn][R][KoS]
     const int tid = threadIdx.x;
     const float2* xn = x + (size_t)n * P * K;
+    for (int i = tid; i < R * 2 * pad; i += 256) {
+        const int r = i / (2 * pad), e = i - r * 2 * pad;
+        xs[r * KS + (e < pad ? e : K + e)] = make_float2(0.f, 0.f);
+    }
 
     // pulse-filter column of this thread and its streaming state
     const bool colok = tid < cn * Ko;
@@ -53,19 +67,16 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
     #pragma unroll
     for (int s = 0; s < NWP; ++s) pacc[s] = make_float2(0.f, 0.f);
     // rows are numbered p = Dp m - plp + ph (period m, phase ph); slot s holds output m - NWP + 1 + s in period m;
-    // the stream starts at the virtual row -plp (m = 0, ph = 0), rows before 0 being zero
-    int pm = 0, pph = 0;
+    // the stream starts at the virtual row -plp (m = 0, ph = 0), rows before 0 being zero. The slots move down by one
+    // from a period to the next with the sums of its first row (acc[s] = h v + acc[s + 1]), not by moves of their own
+    int pm = plp / Dp, pph = plp - pm * Dp;    // row 0: the zero rows before it leave every slot zero
+    for (int d = 0; d <= pm - NWP && d < Po; ++d)      // (outputs that read no other rows)
+        if (colok) zc[(size_t)d * Ko] = make_float2(0.f, 0.f);
     auto end_period = [&]() {
         const int done = pm - NWP + 1;
         if (colok && done >= 0 && done < Po) zc[(size_t)done * Ko] = pacc[0];
-        #pragma unroll
-        for (int s = 0; s < NWP - 1; ++s) pacc[s] = pacc[s + 1];
-        pacc[NWP - 1] = make_float2(0.f, 0.f);
         ++pm;
     };
-    for (int v = 0; v < plp; ++v) {            // the zero rows before row 0
-        if (++pph == Dp) { end_period(); pph = 0; }
-    }
 
     // the first XPF samples per thread of each chunk are loaded a chunk ahead into registers (their latency hidden
     // behind the chunk before), the rest when the chunk is staged
@@ -90,12 +101,12 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
                 const int i = tid + 256 * k;
                 if (i < cnt) {
                     const int r = i / K;
-                    xs[r * KS + (i - r * K)] = xpf[k];
+                    xs[r * KS + pad + (i - r * K)] = xpf[k];
                 }
             }
             for (int i = tid + 256 * XPF; i < cnt; i += 256) {
                 const int r = i / K;
-                xs[r * KS + (i - r * K)] = src[i];
+                xs[r * KS + pad + (i - r * K)] = src[i];
             }
         }
         __syncthreads();
@@ -115,16 +126,19 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
             const int c = tid / R, r = tid - c * R;
             if (r < rn) {
                 constexpr int DL = DK ? DK : DMAX;    // phases the loops run over
-                float hk[DL][NWK];                    // the taps of every phase, uniform (scalar registers)
+                float hk[DL][NWK];                    // the taps of every phase
                 #pragma unroll
                 for (int ph = 0; ph < DL; ++ph) {
                     #pragma unroll
-                    for (int s = 0; s < NWK; ++s) hk[ph][s] = (DK || ph < Dk) ? hk_t[ph * NWK + s] : 0.f;
+                    for (int s = 0; s < NWK; ++s) {
+                        hk[ph][s] = (DK || ph < Dk) ? hk_t[ph * NWK + s] : 0.f;
+                        if (DL * NWK <= VTAPS) in_vgpr(hk[ph][s]);
+                    }
                 }
                 const double a = (double)ra0, b = (double)rb0;
                 float er, ei, wr = 0.f, wi = 0.f;
                 cis_cyc(b, er, ei);
-                const float2* xr = xs + r * KS;
+                const float2* xr = xs + r * KS + pad;
                 float2* yr = ys + ((size_t)c * R + r) * KoS;
                 // ring of accumulators: output o lives in slot o mod NWK; the period loop is unrolled NWK times so
                 // that every slot index is a constant
@@ -142,11 +156,7 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
                             if (kb + (DK ? DK : Dk) > 0 && kb < K) {  // a period with samples in [0, K)
                                 float2 v[DL];
                                 #pragma unroll
-                                for (int ph = 0; ph < DL; ++ph) {
-                                    const int k = kb + ph;
-                                    const float2 t = xr[min(max(k, 0), K - 1)];
-                                    v[ph] = ((DK || ph < Dk) && k >= 0 && k < K) ? t : make_float2(0.f, 0.f);
-                                }
+                                for (int ph = 0; ph < DL; ++ph) v[ph] = xr[kb + (DK ? ph : min(ph, Dk - 1))];
                                 if (m - mseed >= 16) {        // reseed in float64 every 16 periods
                                     cis_cyc(fma((double)kb - kc, b, a), wr, wi);
                                     mseed = m;
@@ -188,7 +198,10 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
         #pragma unroll
         for (int ph = 0; ph < PL; ++ph) {
             #pragma unroll
-            for (int s = 0; s < NWP; ++s) hp[ph][s] = (DP || ph < Dp) ? hp_t[ph * NWP + s] : 0.f;
+            for (int s = 0; s < NWP; ++s) {
+                hp[ph][s] = (DP || ph < Dp) ? hp_t[ph * NWP + s] : 0.f;
+                if (PL * NWP <= VTAPS) in_vgpr(hp[ph][s]);
+            }
         }
         const float2* yc = ys + (size_t)pc * R * KoS + pj;
         for (int r = 0; r < rn; ++r) {
@@ -198,8 +211,9 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
                 if (ph == pph) {
                     #pragma unroll
                     for (int s = 0; s < NWP; ++s) {
-                        pacc[s].x = fmaf(hp[ph][s], v.x, pacc[s].x);
-                        pacc[s].y = fmaf(hp[ph][s], v.y, pacc[s].y);
+                        const float2 o = ph ? pacc[s] : s + 1 < NWP ? pacc[s + 1 < NWP ? s + 1 : s] : make_float2(0.f, 0.f);
+                        pacc[s].x = fmaf(hp[ph][s], v.x, o.x);
+                        pacc[s].y = fmaf(hp[ph][s], v.y, o.y);
                     }
                 }
             }
@@ -209,8 +223,13 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
         // writes ys, which the barrier after that load orders after every thread's pulse filter of this chunk
     }
     // the zero rows after the last: finish the open period, then every period until the last output is stored
-    if (pph != 0) { end_period(); pph = 0; }
-    while (pm - NWP + 1 < Po) end_period();
+    if (pph != 0) end_period();
+    while (pm - NWP + 1 < Po) {
+        #pragma unroll
+        for (int s = 0; s < NWP - 1; ++s) pacc[s] = pacc[s + 1];
+        pacc[NWP - 1] = make_float2(0.f, 0.f);
+        end_period();
+    }
 }
 
 }  // namespace fsh
