@@ -898,7 +898,11 @@ __global__ __launch_bounds__(256) void k_final_tiles(const float2* __restrict__ 
 // own ratios (one complex multiply each); per q the block's A and B rows take BI - 1 multiplies each, then BI^2
 // complex multiply-adds. Each pixel sums its (p, q) terms in order; a lane reads its tile's samples one ahead of
 // their use. W: aperture weights present.
-template <int T, bool W>
+//
+// HS 2: two threads a block, four of its rows each (every entry of the row table formed, four kept), for images whose
+// lanes fill the SIMDs once: one wave a SIMD issues an instruction in about 5.3 cycles, two in 2.7 each, and a half
+// block's sample takes 212 instructions to a whole one's 337. Same sums, same order.
+template <int T, bool W, int HS>
 __global__ __launch_bounds__(256) void k_final_tiles_reg(const float2* __restrict__ data, int B, int Pf, int Qf,
                                                           const double* __restrict__ ux, const double* __restrict__ uy,
                                                           const double* __restrict__ tgeo, double spx, double spy, double a0,
@@ -909,20 +913,21 @@ __global__ __launch_bounds__(256) void k_final_tiles_reg(const float2* __restric
 {
     constexpr int BI = T < 8 ? T : 8;
     constexpr int NB = T / BI;                     // blocks per tile side
+    constexpr int RH = BI / HS;                    // rows a thread
     // SP consecutive lanes (a power of two up to 64) share one pixel block, each summing the subapertures
     // p = sp, sp + SP, ...; the partial sums are added across those lanes in a fixed butterfly order
     const long gid0 = (long)blockIdx.x * 256 + threadIdx.x;
-    const long gid = gid0 / SP;
-    const int sp = (int)(gid0 - gid * SP);
+    const long gidh = gid0 / SP, gid = gidh / HS;
+    const int sp = (int)(gid0 - gidh * SP), hs = (int)(gidh - gid * HS);
     const long b = gid / (NB * NB);
     if (b >= B) return;
     const int blk = (int)(gid - b * NB * NB), bx = blk / NB, by = blk - bx * NB;
     const int i0 = bx * BI, j0 = by * BI;
     const double hc = 0.5 * (T - 1);
     const double dx0 = (i0 - hc) * spx, dy0 = (j0 - hc) * spy;
-    float2 acc[BI][BI];
+    float2 acc[RH][BI];
     #pragma unroll
-    for (int a = 0; a < BI; ++a)
+    for (int a = 0; a < RH; ++a)
         #pragma unroll
         for (int c = 0; c < BI; ++c) acc[a][c] = make_float2(0.f, 0.f);
     const float2* dp = data + (size_t)b * Pf * Qf;
@@ -966,8 +971,12 @@ __global__ __launch_bounds__(256) void k_final_tiles_reg(const float2* __restric
                     bv[k].x *= wb[k]; bv[k].y *= wb[k];
                 }
             }
+            if (HS == 2) {
+                #pragma unroll
+                for (int k = 0; k < RH; ++k) av[k] = hs ? av[RH + (HS == 2 ? k : 0)] : av[k];
+            }
             #pragma unroll
-            for (int a = 0; a < BI; ++a)
+            for (int a = 0; a < RH; ++a)
                 #pragma unroll
                 for (int c = 0; c < BI; ++c) {
                     acc[a][c].x = fmaf(av[a].x, bv[c].x, acc[a][c].x);
@@ -983,7 +992,7 @@ __global__ __launch_bounds__(256) void k_final_tiles_reg(const float2* __restric
     }
     for (int m = 1; m < SP; m <<= 1) {
         #pragma unroll
-        for (int a = 0; a < BI; ++a)
+        for (int a = 0; a < RH; ++a)
             #pragma unroll
             for (int c = 0; c < BI; ++c) {
                 acc[a][c].x += __shfl_xor(acc[a][c].x, m, 64);
@@ -992,10 +1001,10 @@ __global__ __launch_bounds__(256) void k_final_tiles_reg(const float2* __restric
     }
     if (sp != 0) return;
     const double cx = tgeo[3 * b], cy = tgeo[3 * b + 1], f = fc2 / (2.0 * tgeo[3 * b + 2]);
-    const int X0 = tile_xy[2 * b] - ox + i0, Y0 = tile_xy[2 * b + 1] - oy + j0;
+    const int X0 = tile_xy[2 * b] - ox + i0 + hs * RH, Y0 = tile_xy[2 * b + 1] - oy + j0;
     #pragma unroll
-    for (int a = 0; a < BI; ++a) {
-        const double dx = dx0 + a * spx;
+    for (int a = 0; a < RH; ++a) {
+        const double dx = dx0 + (hs * RH + a) * spx;
         #pragma unroll
         for (int c = 0; c < BI; ++c) {
             const int X = X0 + a, Y = Y0 + c;
@@ -1387,16 +1396,25 @@ int launch_final_tiles(const float2* data, int B, int Pf, int Qf, int T, const d
             return launch_final_tiles_mfma(data, B, Pf, Qf, T, ux, uy, tgeo, spx, spy, a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy,
                                            nx, ny, out, s, split);
         const int per = (T / std::min(T, 8)) * (T / std::min(T, 8));
-        const long blocks = ((long)B * per * split + 255) / 256;
+        // two threads a block where the launch's lanes come to at most a wave a SIMD (65,536): beyond, whole blocks
+        const bool half = T >= 8 && (long)B * per * split <= 65536;
+        const long blocks = ((long)B * per * split * (half ? 2 : 1) + 255) / 256;
         const bool w = w0 != nullptr;
-#define FSH_FR(TT, WW) hipLaunchKernelGGL((k_final_tiles_reg<TT, WW>), dim3((unsigned)blocks), dim3(256), 0, s, data, B, Pf, Qf, ux, uy, \
+#define FSH_FR(TT, WW, HH) hipLaunchKernelGGL((k_final_tiles_reg<TT, WW, HH>), dim3((unsigned)blocks), dim3(256), 0, s, data, B, Pf, Qf, ux, uy, \
                                           tgeo, spx, spy, a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy, nx, ny, out, split)
+#define FSH_FR_H(TT)                                                                                                   \
+    do {                                                                                                               \
+        if (half) { if (w) FSH_FR(TT, true, 2); else FSH_FR(TT, false, 2); }                                           \
+        else if (w) FSH_FR(TT, true, 1);                                                                               \
+        else FSH_FR(TT, false, 1);                                                                                     \
+    } while (0)
         switch (T) {
-            case 4: if (w) FSH_FR(4, true); else FSH_FR(4, false); break;
-            case 8: if (w) FSH_FR(8, true); else FSH_FR(8, false); break;
-            case 16: if (w) FSH_FR(16, true); else FSH_FR(16, false); break;
-            default: if (w) FSH_FR(32, true); else FSH_FR(32, false); break;
+            case 4: if (w) FSH_FR(4, true, 1); else FSH_FR(4, false, 1); break;
+            case 8: FSH_FR_H(8); break;
+            case 16: FSH_FR_H(16); break;
+            default: FSH_FR_H(32); break;
         }
+#undef FSH_FR_H
 #undef FSH_FR
         FSH_TRY(hipGetLastError());
         return OK;
