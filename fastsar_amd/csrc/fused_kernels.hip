@@ -92,9 +92,11 @@ bool level_fused_shape(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int 
 }
 
 // whether a former takes the fused form for a level: where one workgroup holds all of a parent's children (the
-// parent's rows are read once) and they cover at least half of its threads; the two-pass form (the matrix-core range
-// filter) where the children are long or many. FSH_LEVEL_KERNEL=fused forces it where it applies, =split or =mfma
-// turns it off.
+// parent's rows are read once) and they cover a quarter of its threads or more; the other forms where the children are
+// long or many. From 64 columns, not 128: a 2048 x 2048 image's level 3 (16,384 parents of 4 x 29 columns) takes 594 us
+// here and 1,200 on the one-pass matrix-core form, whose blocks of 8 children it half fills (and in float32, where that
+// form's range products are bfloat16 x 3). FSH_LEVEL_KERNEL=fused forces it where it applies, =split or =mfma turns it
+// off.
 bool level_fused_preferred(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int Dp)
 {
     int CB, R;
@@ -103,7 +105,7 @@ bool level_fused_preferred(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, 
     const char* force = getenv("FSH_LEVEL_KERNEL");
     if (force && strcmp(force, "fused") == 0) return true;
     if (force && strcmp(force, "mfma") == 0) return false;
-    return CB == C && CB * Ko >= 128;
+    return CB == C && CB * Ko >= 64;
 }
 
 int launch_level_fused(const float2* x, int Np, int P, int K, const float* c0, const float* sl, int C, const float* hk_t,
