@@ -286,12 +286,41 @@ __device__ __forceinline__ void bp_region(const BpArgs& A)
         for (int p0 = 0; p0 < ntb; p0 += NB) {
             const int nb = min(NB, ntb - p0);
             if (p0 > 0) __syncthreads();                   // the previous windows are read
-            for (int k = 0; k < nb; ++k) {                 // the windows, a pulse at a time across the workgroup
-                const int lo = s_lo[p0 + k];
-                const size_t rowp = (size_t)(pt + p0 + k) * A.W;
-                for (int m = tid; m < NWIN; m += 256) {
-                    const int b = lo + m;
-                    s_win[k * NWIN + m] = (b >= 0 && b < A.W) ? prof_at<PT>(A.win, rowp + b) : make_float2(0.f, 0.f);
+            if constexpr (CUBIC) {
+                // the windows, four pulses and two runs of 256 bins a time, eight loads in flight a thread (1024 x 1024 image
+                // from 2,048 pulses 2.82 -> 2.67 ms; linear reads, whose windows are shorter, lose 5 % by it)
+                for (int k0 = 0; k0 < nb; k0 += 4) {
+                    const int nk = min(4, nb - k0);
+                    for (int mh = 0; mh < NWIN; mh += 512) {
+                        float2 v[4][2];
+                        #pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const int k = k0 + min(u, nk - 1), lo = __builtin_amdgcn_readfirstlane(s_lo[p0 + k]);
+                            const size_t rowp = (size_t)(pt + p0 + k) * A.W;
+                            #pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                const int m = mh + 256 * h + tid, b = lo + m;
+                                v[u][h] = make_float2(0.f, 0.f);
+                                if (m < NWIN && (unsigned)b < (unsigned)A.W) v[u][h] = prof_at<PT>(A.win, rowp + b);
+                            }
+                        }
+                        #pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            #pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                const int m = mh + 256 * h + tid;
+                                if (u < nk && m < NWIN) s_win[(k0 + u) * NWIN + m] = v[u][h];
+                            }
+                    }
+                }
+            } else {
+                for (int k = 0; k < nb; ++k) {                 // the windows, a pulse at a time across the workgroup
+                    const int lo = s_lo[p0 + k];
+                    const size_t rowp = (size_t)(pt + p0 + k) * A.W;
+                    for (int m = tid; m < NWIN; m += 256) {
+                        const int b = lo + m;
+                        s_win[k * NWIN + m] = (b >= 0 && b < A.W) ? prof_at<PT>(A.win, rowp + b) : make_float2(0.f, 0.f);
+                    }
                 }
             }
             __syncthreads();
