@@ -24,33 +24,58 @@ namespace fsh {
 
 // x[p, k] = S[p, k] * wp[p] * wk[k] (wp == nullptr: copy); bad: the first pulse holding a NaN or inf. The rows may be
 // a block of a longer history starting at pulse p0 (wp, ramp and the pointers offset by the caller; bad absolute)
-// with xmax: the largest component magnitude of x as well (float bits compared as unsigned, one atomic per wave;
-// a NaN or inf, which the scan reports, is left out)
+// with xmax: the largest component magnitude of x as well (float bits compared as unsigned; a NaN or inf, which the scan
+// reports, is left out): reduced over the block, one atomic a block and only where it raises the maximum (one a wave of
+// 4,096 blocks took 125 us of a 180 x 159 image's 500)
 __device__ __forceinline__ void note_max(float m, unsigned* xmax)
 {
     if (!xmax) return;
+    __shared__ float wmax[4];
     for (int k = 32; k >= 1; k >>= 1) m = fmaxf(m, __shfl_xor(m, k, 64));
-    if ((threadIdx.x & 63) == 0 && m > 0.f) atomicMax(xmax, __float_as_uint(m));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+        if (__float_as_uint(m) > *(volatile unsigned*)xmax) atomicMax(xmax, __float_as_uint(m));
+    }
 }
 
+// Samples a block of the history's first pass takes: a row's run of 1,024, four a thread in flight, row and column from
+// the grid (no division a sample), and the largest component kept to the block's end for at most one atomic. A wave of 64
+// samples that did its own atomic was bound by them: 1,126 x 600 samples with float16 intermediates 134 us, now 32; 8,190 x
+// 3,073 with them 0.243 -> 0.118 ms, 16,384 x 8,192 in float32 0.48 -> 0.41.
+constexpr int PREP_RUN = 1024;
+
+// one sample of the first pass: scanned, re-referenced, windowed and stored; m: the largest component so far
+__device__ __forceinline__ void prepare_sample(float2 v, int p, int k, int K, const float* wp, const float* wk, float2* x,
+                                               int* bad, const double2* ramp, int p0, float& m)
+{
+    if (!(isfinite(v.x) && isfinite(v.y))) atomicMin(bad, p0 + p);
+    v = apply_ramp(v, ramp, p, k);
+    if (wp) {
+        const float g = wp[p] * wk[k];
+        v.x *= g; v.y *= g;
+    }
+    x[(size_t)p * K + k] = v;
+    const float a = fmaxf(fabsf(v.x), fabsf(v.y));
+    if (a < INFINITY) m = fmaxf(m, a);
+}
+
+// grid (P, ceil(K / PREP_RUN)), or fewer and further ones in turn: a block takes runs of single pulses' samples
 __global__ __launch_bounds__(256) void k_prepare(const float2* __restrict__ S, int P, int K, const float* __restrict__ wp,
                                                   const float* __restrict__ wk, float2* __restrict__ x, int* __restrict__ bad,
                                                   unsigned* __restrict__ xmax, const double2* __restrict__ ramp, int p0)
 {
-    const size_t n = (size_t)P * K;
     float m = 0.f;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        float2 v = S[i];
-        const int p = (int)(i / K);
-        if (!(isfinite(v.x) && isfinite(v.y))) atomicMin(bad, p0 + p);
-        v = apply_ramp(v, ramp, p, (int)(i - (size_t)p * K));
-        if (wp) {
-            const float g = wp[p] * wk[i - (size_t)p * K];
-            v.x *= g; v.y *= g;
+    for (int p = blockIdx.x; p < P; p += gridDim.x) {
+        for (long k0 = (long)blockIdx.y * PREP_RUN + threadIdx.x; k0 < K; k0 += (long)gridDim.y * PREP_RUN) {
+            float2 v[PREP_RUN / 256];
+            #pragma unroll
+            for (int u = 0; u < PREP_RUN / 256; ++u) v[u] = S[(size_t)p * K + min(k0 + 256 * u, (long)K - 1)];
+            #pragma unroll
+            for (int u = 0; u < PREP_RUN / 256; ++u)
+                if (k0 + 256 * u < K) prepare_sample(v[u], p, (int)k0 + 256 * u, K, wp, wk, x, bad, ramp, p0, m);
         }
-        x[i] = v;
-        const float a = fmaxf(fabsf(v.x), fabsf(v.y));
-        if (a < INFINITY) m = fmaxf(m, a);
     }
     note_max(m, xmax);
 }
@@ -1035,10 +1060,8 @@ static int lds_limit()
 int launch_prepare(const float2* S, int P, int K, const float* wp, const float* wk, float2* x, int* bad, hipStream_t s,
                    unsigned* xmax, const double* ramp, int p0)
 {
-    const size_t n = (size_t)P * K;
-    // with xmax, 4096 blocks (enough to keep HBM busy) so that the one atomic per wave stays a few thousand
-    const int blocks = (int)std::min<size_t>((n + 255) / 256, xmax ? 4096 : 1 << 16);
-    hipLaunchKernelGGL(k_prepare, dim3(blocks), dim3(256), 0, s, S, P, K, wp, wk, x, bad, xmax, (const double2*)ramp, p0);
+    const dim3 grid((unsigned)std::min(P, 1 << 20), (unsigned)std::min((K - 1) / PREP_RUN + 1, 65535));
+    hipLaunchKernelGGL(k_prepare, grid, dim3(256), 0, s, S, P, K, wp, wk, x, bad, xmax, (const double2*)ramp, p0);
     FSH_TRY(hipGetLastError());
     return OK;
 }
@@ -1078,20 +1101,16 @@ __global__ __launch_bounds__(256) void k_prepare16(const void* __restrict__ S, i
                                                     float2* __restrict__ x, int* __restrict__ bad, unsigned* __restrict__ xmax,
                                                     const double2* __restrict__ ramp, int p0)
 {
-    const size_t n = (size_t)P * K;
     float m = 0.f;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int p = (int)(i / K);
-        float2 v = decode_sample<DT>(S, i, inv, p);
-        if (!(isfinite(v.x) && isfinite(v.y))) atomicMin(bad, p0 + p);
-        v = apply_ramp(v, ramp, p, (int)(i - (size_t)p * K));
-        if (wp) {
-            const float g = wp[p] * wk[i - (size_t)p * K];
-            v.x *= g; v.y *= g;
+    for (int p = blockIdx.x; p < P; p += gridDim.x) {
+        for (long k0 = (long)blockIdx.y * PREP_RUN + threadIdx.x; k0 < K; k0 += (long)gridDim.y * PREP_RUN) {
+            float2 v[PREP_RUN / 256];
+            #pragma unroll
+            for (int u = 0; u < PREP_RUN / 256; ++u) v[u] = decode_sample<DT>(S, (size_t)p * K + min(k0 + 256 * u, (long)K - 1), inv, p);
+            #pragma unroll
+            for (int u = 0; u < PREP_RUN / 256; ++u)
+                if (k0 + 256 * u < K) prepare_sample(v[u], p, (int)k0 + 256 * u, K, wp, wk, x, bad, ramp, p0, m);
         }
-        x[i] = v;
-        const float a = fmaxf(fabsf(v.x), fabsf(v.y));
-        if (a < INFINITY) m = fmaxf(m, a);
     }
     note_max(m, xmax);
 }
@@ -1122,19 +1141,18 @@ int launch_half_scales(const unsigned* xmax, const float* gain, int n, float* hs
 int launch_prepare16(const void* S, int dtype, const float* inv, int P, int K, const float* wp, const float* wk, float2* x,
                      int* bad, hipStream_t s, unsigned* xmax, const double* ramp, int p0)
 {
-    const size_t n = (size_t)P * K;
-    const int blocks = (int)std::min<size_t>((n + 255) / 256, xmax ? 4096 : 1 << 16);
+    const dim3 grid((unsigned)std::min(P, 1 << 20), (unsigned)std::min((K - 1) / PREP_RUN + 1, 65535));
     if (dtype == 1)
-        hipLaunchKernelGGL(k_prepare16<1>, dim3(blocks), dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
+        hipLaunchKernelGGL(k_prepare16<1>, grid, dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
                            (const double2*)ramp, p0);
     else if (dtype == 2)
-        hipLaunchKernelGGL(k_prepare16<2>, dim3(blocks), dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
+        hipLaunchKernelGGL(k_prepare16<2>, grid, dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
                            (const double2*)ramp, p0);
     else if (dtype == 3)
-        hipLaunchKernelGGL(k_prepare16<3>, dim3(blocks), dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
+        hipLaunchKernelGGL(k_prepare16<3>, grid, dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
                            (const double2*)ramp, p0);
     else if (dtype == 4)
-        hipLaunchKernelGGL(k_prepare16<4>, dim3(blocks), dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
+        hipLaunchKernelGGL(k_prepare16<4>, grid, dim3(256), 0, s, S, P, K, inv, wp, wk, x, bad, xmax,
                            (const double2*)ramp, p0);
     else {
         set_error("prepare: unknown history type");
