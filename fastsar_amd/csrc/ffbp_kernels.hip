@@ -760,18 +760,20 @@ __global__ __launch_bounds__(256) void k_device_phases(const double* __restrict_
 
 // ------------------------------------------------------------------------------------------------ final geometry
 
-// grid B tiles, block 256: ux, uy [B, Pf] (float64) and per tile (ucx, ucy, rc) [B, 3]
+// a wave a tile, four tiles a block: ux, uy [B, Pf] (float64) and per tile (ucx, ucy, rc) [B, 3], the sums over the
+// subapertures by shuffles. (A block of 256 threads a tile left most of them idle at 24 to 80 subapertures and met eight
+// times in LDS: 65,536 tiles of 44 subapertures 83 us, 336,000 of 24 400 us.)
 __global__ __launch_bounds__(256) void k_final_geom(const double* __restrict__ fu, const double* __restrict__ fr0,
-                                                     const double* __restrict__ cen, int Pf, double e1x, double e1y, double e1z,
-                                                     double e2x, double e2y, double e2z, double* __restrict__ ux,
+                                                     const double* __restrict__ cen, int B, int Pf, double e1x, double e1y,
+                                                     double e1z, double e2x, double e2y, double e2z, double* __restrict__ ux,
                                                      double* __restrict__ uy, double* __restrict__ tgeo)
 {
-    __shared__ double red[4][256];
-    const int b = blockIdx.x, tid = threadIdx.x;
+    const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (b >= B) return;
     const double enx = e1y * e2z - e1z * e2y, eny = e1z * e2x - e1x * e2z, enz = e1x * e2y - e1y * e2x;
-    const double cx = cen[3 * b], cy = cen[3 * b + 1], cz = cen[3 * b + 2];
+    const double cx = cen[3 * (size_t)b], cy = cen[3 * (size_t)b + 1], cz = cen[3 * (size_t)b + 2];
     double sx = 0.0, sy = 0.0, sz = 0.0, sw = 0.0;
-    for (int p = tid; p < Pf; p += 256) {
+    for (int p = lane; p < Pf; p += 64) {
         const double wx = fr0[p] * fu[3 * p] - cx, wy = fr0[p] * fu[3 * p + 1] - cy, wz = fr0[p] * fu[3 * p + 2] - cz;
         const double wn = sqrt(wx * wx + wy * wy + wz * wz);
         const double a = (wx * e1x + wy * e1y + wz * e1z) / wn;
@@ -781,19 +783,18 @@ __global__ __launch_bounds__(256) void k_final_geom(const double* __restrict__ f
         uy[(size_t)b * Pf + p] = c;
         sx += a; sy += c; sz += e; sw += wn;
     }
-    red[0][tid] = sx; red[1][tid] = sy; red[2][tid] = sz; red[3][tid] = sw;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s)
-            for (int k = 0; k < 4; ++k) red[k][tid] += red[k][tid + s];
-        __syncthreads();
+    for (int m = 32; m >= 1; m >>= 1) {
+        sx += __shfl_xor(sx, m, 64);
+        sy += __shfl_xor(sy, m, 64);
+        sz += __shfl_xor(sz, m, 64);
+        sw += __shfl_xor(sw, m, 64);
     }
-    if (tid == 0) {
-        const double mx = red[0][0] / Pf, my = red[1][0] / Pf, mz = red[2][0] / Pf;
+    if (lane == 0) {
+        const double mx = sx / Pf, my = sy / Pf, mz = sz / Pf;
         const double mn = sqrt(mx * mx + my * my + mz * mz);
-        tgeo[3 * b] = mx / mn;
-        tgeo[3 * b + 1] = my / mn;
-        tgeo[3 * b + 2] = red[3][0] / Pf;
+        tgeo[3 * (size_t)b] = mx / mn;
+        tgeo[3 * (size_t)b + 1] = my / mn;
+        tgeo[3 * (size_t)b + 2] = sw / Pf;
     }
 }
 
@@ -1368,7 +1369,7 @@ int launch_final_geom(const double* fu, const double* fr0, const double* cen, in
                       double* ux, double* uy, double* tgeo, hipStream_t s)
 {
     if (B < 1 || Pf < 1) { set_error("final_geom: invalid shape"); return E_INVALID; }
-    hipLaunchKernelGGL(k_final_geom, dim3(B), dim3(256), 0, s, fu, fr0, cen, Pf, e1[0], e1[1], e1[2], e2[0], e2[1], e2[2], ux,
+    hipLaunchKernelGGL(k_final_geom, dim3((unsigned)(((long)B + 3) / 4)), dim3(256), 0, s, fu, fr0, cen, B, Pf, e1[0], e1[1], e1[2], e2[0], e2[1], e2[2], ux,
                        uy, tgeo);
     FSH_TRY(hipGetLastError());
     return OK;
