@@ -182,4 +182,193 @@ int launch_final_tiles_mfma(const float2* data, int B, int Pf, int Qf, int T, co
     return OK;
 }
 
+// 32 x 32 tiles with each pixel's terms in the order of k_final_tiles_reg, bit for bit: a wave holds a tile's sums over the
+// subapertures p = sp, sp + SP, ... and adds two samples' terms an instruction (contraction index: sample, then real and
+// imaginary part; the instruction is an ascending chain of fused multiply-adds). The wave's lanes build eight samples'
+// tables of one subaperture at a time, eight runs x eight samples, each lane from its own sample's ratio and first entry,
+// advanced eight products a chunk; seeds for eight subapertures at once.
+//
+// One 8 x 8 block a lane took 337 instructions for 256 multiply-adds and, at 1.1 to 2 waves a SIMD, waited for half of
+// them; here 1,024 pixels share tables of 64 entries a sample and the launch runs 4.5 waves a SIMD at 2,304 tiles with
+// two waves each. Final stage of 1,536 x 1,536 pixels (116 x 78 samples a tile) 3.50 -> 1.88 ms, 2,048 x 2,048 (118 x 77)
+// 5.69 -> 3.14, 3,000 x 2,500 8.9 -> 6.3, 8,192 x 8,192 59 -> 44 (101 TFLOP/s of the float32 rate's 154): faster at every
+// size, so no 32 x 32 tile takes the register form. Bound by the matrix pipe (1,120 cycles a chunk) and the tables'
+// VALU instructions (about 500) in turn. v_mfma_f32_32x32x2_f32, a sample an instruction: 1.95 ms, 44.5.
+namespace {
+struct OrderShape {
+    static constexpr int RS = 65;                            // row stride of the tables (float2): writes free of conflicts
+    static constexpr int TAB = 8 * RS;                       // [8 samples][32 rows of A, 32 columns of B]
+    static constexpr int SEED = 4 * 64;                      // seeds of 8 subapertures x 8 runs
+    static constexpr int ESZ = 1024;                         // float2 a wave: tables and seeds, then the sums
+    static_assert(TAB + SEED <= ESZ, "a wave's tables and seeds fit its sums' room");
+};
+}  // namespace
+
+template <bool W>
+__global__ __launch_bounds__(256) void k_final_tiles_order(const float2* __restrict__ data, int B, int Pf, int Qf,
+                                                            const double* __restrict__ ux, const double* __restrict__ uy,
+                                                            const double* __restrict__ tgeo, double spx, double spy, double a0,
+                                                            double a1, double fc2, const float* __restrict__ w0,
+                                                            const float* __restrict__ gx, const float* __restrict__ gyr,
+                                                            const int* __restrict__ tile_xy, int ox, int oy, int nx, int ny,
+                                                            float2* __restrict__ out, int SP)
+{
+    typedef OrderShape S;
+    constexpr int T = 32;
+    __shared__ float2 lds[4 * S::ESZ];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int sp = wv & (SP - 1);                            // SP 1, 2 or 4 waves a tile
+    const long bt = (long)blockIdx.x * (4 / SP) + wv / SP;
+    const bool live = bt < B;
+    const int b = (int)(live ? bt : B - 1);
+    const double hc = 0.5 * (T - 1);
+    // table role: run of 8 entries (0 .. 3 A's rows, 4 .. 7 B's columns), sample qi of the chunk's 8
+    const int run = lane >> 3, qi = lane & 7;
+    const bool isA = run < 4;
+    const double spc = isA ? spx : spy, dl0 = (8 * (run & 3) - hc) * spc;
+    const double* gp = (isA ? ux : uy) + (size_t)b * Pf;
+    float2* E = lds + wv * S::ESZ;
+    float2* sd = E + S::TAB;
+    float2* ew = E + qi * S::RS + 8 * run;
+    // product role: row or column i; contraction index k: sample k / 2 of the two, component k % 2
+    const int i = lane & 15, k = lane >> 4, comp = k & 1;
+    const float* ea = (const float*)(E + (k >> 1) * S::RS + i) + comp;
+    const float* er = (const float*)(E + (k >> 1) * S::RS + 32 + i) + comp;
+    const float* ei = (const float*)(E + (k >> 1) * S::RS + 32 + i) + (comp ^ 1);
+    const unsigned neg = comp ? 0x80000000u : 0u;            // re: Ax Bx - Ay By
+    floatx4_t re[2][2], im[2][2];
+    #pragma unroll
+    for (int m = 0; m < 2; ++m)
+        #pragma unroll
+        for (int n = 0; n < 2; ++n) re[m][n] = im[m][n] = floatx4_t{};
+
+    for (int pg = sp; pg < Pf; pg += 8 * SP) {
+        {   // seeds of the group's eight subapertures, one a lane and run
+            const double g = gp[min(pg + qi * SP, Pf - 1)];
+            float2 v;
+            wave_lds_sync();
+            cis_cyc(-(g * spc) * a0, v.x, v.y);              // ratio along the run at q = 0
+            sd[4 * lane] = v;
+            cis_cyc(-(g * spc) * a1, v.x, v.y);              // its step over q
+            sd[4 * lane + 1] = v;
+            cis_cyc(-(g * dl0) * a0, v.x, v.y);              // the run's first entry, q = 0
+            sd[4 * lane + 2] = v;
+            cis_cyc(-(g * dl0) * a1, v.x, v.y);
+            sd[4 * lane + 3] = v;
+            wave_lds_sync();
+        }
+        for (int j = 0; j < 8 && pg + j * SP < Pf; ++j) {
+            const size_t bp = (size_t)b * Pf + pg + j * SP;
+            const float2* dq = data + bp * Qf;
+            float2 dn = load_ahead(dq + min(qi, Qf - 1));    // the lane's sample, read one chunk ahead
+            const float2* sj = sd + 4 * (8 * run + j);
+            float2 r = sj[0], ba = sj[2];
+            const float2 sr = sj[1], sb = sj[3];
+            float wt[8];
+            if (W) {
+                const float c0 = isA ? w0[bp] : 1.f, c1 = (isA ? gx : gyr)[bp];
+                #pragma unroll
+                for (int e = 0; e < 8; ++e) wt[e] = c0 + c1 * (float)(dl0 + e * spc);
+            }
+            #pragma unroll
+            for (int t = 0; t < 7; ++t) {                    // to the lane's sample, by the same products
+                const float2 r1 = cmul(r, sr), b1 = cmul(ba, sb);
+                r.x = t < qi ? r1.x : r.x;
+                r.y = t < qi ? r1.y : r.y;
+                ba.x = t < qi ? b1.x : ba.x;
+                ba.y = t < qi ? b1.y : ba.y;
+            }
+            for (int q0 = 0; q0 < Qf; q0 += 8) {
+                // B's lanes take 1 in the sample's place; A's entries past the last sample are 0
+                const float2 z = q0 + qi < Qf ? dn : make_float2(0.f, 0.f);
+                float2 v = cmul(isA ? z : make_float2(1.f, 0.f), ba);
+                dn = load_ahead(dq + min(q0 + 8 + qi, Qf - 1));
+                #pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    ew[e] = W ? make_float2(v.x * wt[e], v.y * wt[e]) : v;
+                    if (e < 7) v = cmul(v, r);
+                }
+                if (q0 + 8 < Qf) {
+                    #pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        r = cmul(r, sr);
+                        ba = cmul(ba, sb);
+                    }
+                }
+                wave_lds_sync();
+                #pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    if (q0 + 2 * s < Qf) {
+                        float a[2], cr[2], ci[2];
+                        #pragma unroll
+                        for (int m = 0; m < 2; ++m) {
+                            a[m] = ea[4 * s * S::RS + 32 * m];
+                            cr[m] = __uint_as_float(__float_as_uint(er[4 * s * S::RS + 32 * m]) ^ neg);
+                            ci[m] = ei[4 * s * S::RS + 32 * m];
+                        }
+                        #pragma unroll
+                        for (int m = 0; m < 2; ++m)
+                            #pragma unroll
+                            for (int n = 0; n < 2; ++n) {
+                                re[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m], cr[n], re[m][n], 0, 0, 0);
+                                im[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m], ci[n], im[m][n], 0, 0, 0);
+                            }
+                    }
+                }
+                wave_lds_sync();
+            }
+        }
+    }
+    // the waves of a tile add their sums in k_final_tiles_reg's order (neighbours first)
+    for (int m = 1; m < SP; m <<= 1) {
+        __syncthreads();
+        float2* mine = lds + wv * S::ESZ + lane;
+        if (sp & m) {
+            #pragma unroll
+            for (int u = 0; u < 16; ++u)
+                mine[64 * u] = make_float2(re[u >> 3][u >> 2 & 1][u & 3], im[u >> 3][u >> 2 & 1][u & 3]);
+        }
+        __syncthreads();
+        if (!(sp & m)) {
+            const float2* o = mine + m * S::ESZ;
+            #pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                re[u >> 3][u >> 2 & 1][u & 3] += o[64 * u].x;
+                im[u >> 3][u >> 2 & 1][u & 3] += o[64 * u].y;
+            }
+        }
+    }
+    if (sp || !live) return;
+    const double cx = tgeo[3 * b], cy = tgeo[3 * b + 1], f = fc2 / (2.0 * tgeo[3 * b + 2]);
+    const int X0 = tile_xy[2 * b] - ox, Y0 = tile_xy[2 * b + 1] - oy;
+    #pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int pi = 16 * (u >> 3) + 4 * k + (u & 3), pj = 16 * (u >> 2 & 1) + i, X = X0 + pi, Y = Y0 + pj;
+        if (X < 0 || X >= nx || Y < 0 || Y >= ny) continue;
+        const double dx = (8 * (pi >> 3) - hc) * spx + (pi & 7) * spx, dy = (8 * (pj >> 3) - hc) * spy + (pj & 7) * spy;
+        const double los = cx * dx + cy * dy;
+        float cs, sn;
+        cis_cyc((dx * dx + dy * dy - los * los) * f, cs, sn);
+        out[(size_t)X * ny + Y] = cmul(make_float2(re[u >> 3][u >> 2 & 1][u & 3], im[u >> 3][u >> 2 & 1][u & 3]),
+                                       make_float2(cs, sn));
+    }
+}
+
+int launch_final_tiles_order(const float2* data, int B, int Pf, int Qf, const double* ux, const double* uy, const double* tgeo,
+                             double spx, double spy, double a0, double a1, double fc2, const float* w0, const float* gx,
+                             const float* gyr, const int* tile_xy, int ox, int oy, int nx, int ny, float2* out, hipStream_t s,
+                             int split)
+{
+    if (split < 1 || split > 4) { set_error("final_tiles: one, two or four waves a tile"); return E_INVALID; }
+    const long G = ((long)B * split + 3) / 4;
+    if (w0)
+        hipLaunchKernelGGL(k_final_tiles_order<true>, dim3((unsigned)G), dim3(256), 0, s, data, B, Pf, Qf, ux, uy, tgeo, spx, spy,
+                           a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy, nx, ny, out, split);
+    else
+        hipLaunchKernelGGL(k_final_tiles_order<false>, dim3((unsigned)G), dim3(256), 0, s, data, B, Pf, Qf, ux, uy, tgeo, spx, spy,
+                           a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy, nx, ny, out, split);
+    FSH_TRY(hipGetLastError());
+    return OK;
+}
+
 }  // namespace fsh

@@ -91,6 +91,11 @@ int launch_final_tiles_mfma(const float2* data, int B, int Pf, int Qf, int T, co
                             const double* tgeo, double spx, double spy, double a0, double a1, double fc2, const float* w0,
                             const float* gx, const float* gyr, const int* tile_xy, int ox, int oy, int nx, int ny, float2* out,
                             hipStream_t s, int split);
+// the same for 32 x 32 tiles, each pixel's terms in the register form's order: split 1, 2 or 4 waves a tile
+int launch_final_tiles_order(const float2* data, int B, int Pf, int Qf, const double* ux, const double* uy, const double* tgeo,
+                             double spx, double spy, double a0, double a1, double fc2, const float* w0, const float* gx,
+                             const float* gyr, const int* tile_xy, int ox, int oy, int nx, int ny, float2* out, hipStream_t s,
+                             int split);
 // subapertures summed by separate lanes per pixel block in the final stage: more threads where the image has few
 // tiles (a power of two, 1 for 65536 pixel blocks and more)
 int final_split(long tiles, int T);
