@@ -477,6 +477,7 @@ struct Exact {
     float2* image = nullptr;         // [nseg, nx, ny]
     int nseg = 1;                    // images the pulses of each chunk are dealt to (bp_segments)
     int* bad = nullptr;
+    int* bad_host = nullptr;         // its value after a call (pinned)
     hipfftHandle plan = 0;
     int plan_n = 0;
     bool have_plan = false;
@@ -487,6 +488,7 @@ struct Exact {
         dev_free(ant); dev_free(ref); dev_free(cen); dev_free(blo); dev_free(wp); dev_free(wk); dev_free(hist);
         dev_free(pad); dev_free(prof); dev_free(win); dev_free(winh); dev_free(smax); dev_free(pinv); dev_free(image); dev_free(bad);
         dev_free(ramp);
+        if (bad_host) (void)hipHostFree(bad_host);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -690,7 +692,8 @@ int fsh_exact_create(const fsh_exact_desc* desc, void** handle)
     if ((st = dev_alloc((void**)&e->pad, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->prof, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->win, (size_t)ch * d.W * sizeof(float2))) ||
-        (st = dev_alloc((void**)&e->image, (size_t)e->nseg * d.nx * d.ny * sizeof(float2))) || (st = dev_alloc((void**)&e->bad, sizeof(int))))
+        (st = dev_alloc((void**)&e->image, (size_t)e->nseg * d.nx * d.ny * sizeof(float2))) || (st = dev_alloc((void**)&e->bad, sizeof(int))) ||
+        (st = pinned_int(&e->bad_host)))
         return fail(st);
     if (d.profiles && ((st = dev_alloc(&e->winh, (size_t)ch * d.W * (d.profiles == 2 ? 8 : 4))) ||
                        (st = dev_alloc((void**)&e->smax, sizeof(unsigned)))))
@@ -775,11 +778,11 @@ static int exact_form_impl(Exact* e, const void* S, int dtype, const float* puls
                            e->image, n, e->nseg, e->image);
         FSH_TRY(hipGetLastError());
     }
-    int badh = INT_MAX;
-    FSH_TRY(hipMemcpyAsync(&badh, e->bad, sizeof(int), hipMemcpyDeviceToHost, e->stream));
+    if ((st = launch_publish_int(e->bad, e->bad_host, e->stream))) return st;
     FSH_TRY(hipMemcpyAsync(image, e->image, (size_t)d.nx * d.ny * sizeof(float2),
                            image_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, e->stream));
     FSH_TRY(hipStreamSynchronize(e->stream));
+    const int badh = *(volatile int*)e->bad_host;
     if (badh != INT_MAX) {
         if (bad_pulse) *bad_pulse = badh;
         char buf[200];

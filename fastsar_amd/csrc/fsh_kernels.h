@@ -16,6 +16,9 @@ int check_history_type(int dtype, const void* pulse_scale);
 int launch_prepare16(const void* S, int dtype, const float* inv, int P, int K, const float* wp, const float* wk, float2* x,
                      int* bad, hipStream_t s, unsigned* xmax = nullptr, const double* ramp = nullptr, int p0 = 0);
 int launch_fill_int(int* p, int n, int value, hipStream_t s);
+// a device word stored into pinned host memory, read there once the stream has been waited for
+int launch_publish_int(const int* src, int* pinned, hipStream_t s);
+int pinned_int(int** p);
 // deferred != nullptr: the caller's pulse filter can apply rho (a launch_fir_p with the same c0, sl, D, pl, kc), and
 // *deferred tells whether the chosen kernel left it out of y; that kernel (the row form) then writes rows ys samples
 // apart (ys >= Ko; 0: Ko), the others always Ko apart
