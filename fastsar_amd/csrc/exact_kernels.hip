@@ -187,14 +187,6 @@ struct BpArgs {
     float2* out;
 };
 
-template <int PT>
-__device__ __forceinline__ float2 prof_at(const void* w, size_t i)
-{
-    if (PT == 0) return static_cast<const float2*>(w)[i];
-    const half2_t h = static_cast<const half2_t*>(w)[PT == 2 ? 2 * i : i];
-    return make_float2((float)h.x, (float)h.y);
-}
-
 template <int BR, int TX, int TY, int PT, bool CUBIC>
 __device__ __forceinline__ void bp_region(const BpArgs& A)
 {
@@ -224,7 +216,10 @@ __device__ __forceinline__ void bp_region(const BpArgs& A)
     // ranges, whose bins (several apart from column to column) fall on different banks, and pixels at one range read the
     // same words. With e1 across range and the lanes along e2 (32 ranges a read, two rows of them) the reads lost 47 % of
     // their LDS cycles to conflicts, LDS busy 65 % of the time
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    typedef typename std::conditional<PT == 0, float2, half2_t>::type Raw;
+    constexpr unsigned ES = PT == 2 ? 2 : 1;           // stored elements a sample
+    const Raw* win = static_cast<const Raw*>(A.win);
     const int col = A.along_e1 ? (tid >> 3) % BR : tid % BR;
     const int row = A.along_e1 ? (tid & 7) + 8 * (tid / (8 * BR)) : tid / BR;
 
@@ -286,42 +281,41 @@ __device__ __forceinline__ void bp_region(const BpArgs& A)
         for (int p0 = 0; p0 < ntb; p0 += NB) {
             const int nb = min(NB, ntb - p0);
             if (p0 > 0) __syncthreads();                   // the previous windows are read
-            if constexpr (CUBIC) {
-                // the windows, four pulses and two runs of 256 bins a time, eight loads in flight a thread (1024 x 1024 image
-                // from 2,048 pulses 2.82 -> 2.67 ms; linear reads, whose windows are shorter, lose 5 % by it)
-                for (int k0 = 0; k0 < nb; k0 += 4) {
-                    const int nk = min(4, nb - k0);
-                    for (int mh = 0; mh < NWIN; mh += 512) {
-                        float2 v[4][2];
-                        #pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const int k = k0 + min(u, nk - 1), lo = __builtin_amdgcn_readfirstlane(s_lo[p0 + k]);
-                            const size_t rowp = (size_t)(pt + p0 + k) * A.W;
-                            #pragma unroll
-                            for (int h = 0; h < 2; ++h) {
-                                const int m = mh + 256 * h + tid, b = lo + m;
-                                v[u][h] = make_float2(0.f, 0.f);
-                                if (m < NWIN && (unsigned)b < (unsigned)A.W) v[u][h] = prof_at<PT>(A.win, rowp + b);
-                            }
-                        }
-                        #pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            #pragma unroll
-                            for (int h = 0; h < 2; ++h) {
-                                const int m = mh + 256 * h + tid;
-                                if (u < nk && m < NWIN) s_win[(k0 + u) * NWIN + m] = v[u][h];
-                            }
+            // the windows: a wave takes every fourth pulse's, four runs of 64 bins in flight, with scalar addresses where the
+            // four lie inside their profiles. The kernel is bound by VALU instructions (24 a pixel and pulse with linear
+            // reads, 3.6 cycles each), and a thread's own address and bounds for every bin were 4 more: 2,001 x 1,603 pixels
+            // from 4,001 pulses, linear, 10.38 -> 9.69 ms; cubic of 181 x 2,347 383 -> 356 us, of 1,024 x 1,024 unchanged.
+            // Eight runs in flight: 10.33 ms, 1,024 x 1,024 2.66 -> 2.83
+            constexpr int U = 4;
+            const int los = s_lo[p0 + min(lane, nb - 1)];      // NB is at most 32
+            for (int k = wv, h = 0; k < nb;) {
+                int kk[U], hh[U], c[U];
+                bool in = true;
+                #pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    kk[u] = k;
+                    hh[u] = h;
+                    c[u] = __builtin_amdgcn_readlane(los, min(k, nb - 1)) + h;
+                    in = in && c[u] >= 0 && c[u] + 64 <= A.W;
+                    h += 64;
+                    if (h >= NWIN) { h = 0; k += 4; }
+                }
+                Raw v[U];
+                if (in) {
+                    #pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        v[u] = (win + (size_t)ES * ((size_t)(pt + p0 + min(kk[u], nb - 1)) * A.W + c[u]))[ES * lane];
+                } else {
+                    #pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int b = c[u] + lane;
+                        v[u] = Raw{};
+                        if ((unsigned)b < (unsigned)A.W) v[u] = win[(size_t)ES * ((size_t)(pt + p0 + min(kk[u], nb - 1)) * A.W + b)];
                     }
                 }
-            } else {
-                for (int k = 0; k < nb; ++k) {                 // the windows, a pulse at a time across the workgroup
-                    const int lo = s_lo[p0 + k];
-                    const size_t rowp = (size_t)(pt + p0 + k) * A.W;
-                    for (int m = tid; m < NWIN; m += 256) {
-                        const int b = lo + m;
-                        s_win[k * NWIN + m] = (b >= 0 && b < A.W) ? prof_at<PT>(A.win, rowp + b) : make_float2(0.f, 0.f);
-                    }
-                }
+                #pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (kk[u] < nb && hh[u] + lane < NWIN) s_win[kk[u] * NWIN + hh[u] + lane] = make_float2((float)v[u].x, (float)v[u].y);
             }
             __syncthreads();
             for (int k = 0; k < nb; ++k) {
