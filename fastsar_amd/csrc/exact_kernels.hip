@@ -686,9 +686,14 @@ int fsh_exact_create(const fsh_exact_desc* desc, void** handle)
     if ((st = dev_alloc((void**)&e->pad, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->prof, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->win, (size_t)ch * d.W * sizeof(float2))) ||
-        (st = dev_alloc((void**)&e->image, (size_t)e->nseg * d.nx * d.ny * sizeof(float2))) || (st = dev_alloc((void**)&e->bad, sizeof(int))) ||
-        (st = pinned_int(&e->bad_host)))
+        (st = dev_alloc((void**)&e->bad, sizeof(int))) || (st = pinned_int(&e->bad_host)))
         return fail(st);
+    st = dev_alloc((void**)&e->image, (size_t)e->nseg * d.nx * d.ny * sizeof(float2));
+    if (st == E_NOMEM && e->nseg > 1) {                    // one image where several do not fit
+        e->nseg = 1;
+        st = dev_alloc((void**)&e->image, (size_t)d.nx * d.ny * sizeof(float2));
+    }
+    if (st) return fail(st);
     if (d.profiles && ((st = dev_alloc(&e->winh, (size_t)ch * d.W * (d.profiles == 2 ? 8 : 4))) ||
                        (st = dev_alloc((void**)&e->smax, sizeof(unsigned)))))
         return fail(st);

@@ -23,3 +23,15 @@ def test_pulses_dealt_to_images(nx, ny, P, interp):
     e = oracle.plain_db(a, b)
     print(f'{nx} x {ny} from {P} {interp}: {e:.1f} dB')
     assert e < -120, e
+
+
+def test_one_image_where_several_do_not_fit(monkeypatch):
+    rng = np.random.default_rng(3)
+    col = sim.spotlight(1024, 256, 2.0)
+    S = (rng.standard_normal((1024, 256)) + 1j * rng.standard_normal((1024, 256))).astype(np.complex64)
+    args = (col.ant, col.fmin, col.df, 256, 64, 65, 0.5, 0.5, (0.0, 1.0, 0.0), (1.0, 0.0, 0.0))
+    a = ExactFormer(*args)(S)
+    monkeypatch.setenv('FSH_FAIL_ALLOC_SIZE', str(16 * 64 * 65 * 8))
+    b = ExactFormer(*args)(S)
+    monkeypatch.delenv('FSH_FAIL_ALLOC_SIZE')
+    assert oracle.plain_db(a, b) < -120 and not np.array_equal(a, b)
