@@ -70,8 +70,8 @@ int launch_level_mfma(const float2* x, int Np, int P, int K, const float* c0, co
 // the same with the decimation factors fixed at (Dk, Dp) = (2, 2), (2, 3), (3, 2), (3, 3) (fused_kernels_k<Dk>p<Dp>.hip),
 // on a shape launch_level_fused has checked
 #define FSH_FUSED_FIXED_DECL(name)                                                                                    \
-    int name(dim3 grid, size_t lds, hipStream_t s, int NWK, int NWP, const float2* x, int P, int K, const float* c0,    \
-             const float* sl, int C, const float* hk_t, int plk, int Ko, const float* hp_t, int plp, int Po, double kc, \
+    int name(dim3 grid, dim3 block, size_t lds, hipStream_t s, int NWK, int NWP, const float2* x, int P, int K,         \
+             const float* c0, const float* sl, int C, const float* hk_t, int plk, int Ko, const float* hp_t, int plp, int Po, double kc, \
              int Np, int CB, int R, float2* z);
 FSH_FUSED_FIXED_DECL(launch_level_fused_k2p2)
 FSH_FUSED_FIXED_DECL(launch_level_fused_k2p3)

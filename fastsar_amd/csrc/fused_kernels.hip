@@ -7,8 +7,8 @@
 //   z_c[i, j] = sum_{r < Lp} hp[r] y_c[Dp i + r - plp, j]
 // with x zero outside [0, K) and y zero outside [0, P).
 //
-// One workgroup of 256 threads takes one parent and a block of CB of its children, and walks the parent's pulses in
-// chunks of R rows:
+// One workgroup of 256 threads (128 where a level has many parents of few columns) takes one parent and a block of CB of
+// its children, and walks the parent's pulses in chunks of R rows:
 //   1. the chunk of x rows [R, K] is loaded with coalesced reads into LDS;
 //   2. one thread per (child, row) streams the row through the range filter: each sample is rotated (a float32
 //      recurrence reseeded in float64 every 32 samples) and added into the NWK = ceil(Lk / Dk) outputs whose taps
@@ -93,7 +93,7 @@ bool level_fused_shape(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int 
 
 // whether a former takes the fused form for a level: where one workgroup holds all of a parent's children (the
 // parent's rows are read once) and they cover a quarter of its threads or more; the other forms where the children are
-// long or many. From 64 columns, not 128: a 2048 x 2048 image's level 3 (16,384 parents of 4 x 29 columns) takes 594 us
+// long or many. From 64 columns, not 128: a 2048 x 2048 image's level 3 (16,384 parents of 4 x 29 columns) takes 440 us
 // here and 1,200 on the one-pass matrix-core form, whose blocks of 8 children it half fills (and in float32, where that
 // form's range products are bfloat16 x 3). FSH_LEVEL_KERNEL=fused forces it where it applies, =split or =mfma turns it
 // off.
@@ -137,13 +137,23 @@ int launch_level_fused(const float2* x, int Np, int P, int K, const float* c0, c
             lds = per_row * R;
         }
     }
-    const dim3 grid((unsigned)G), block(256);
+    // many parents of at most 128 columns: two waves a block, not four of which two would idle through the pulse filter,
+    // and rows for one wave's range filter, so that seven or eight blocks share a CU: 16,384 parents of 4 x 29 columns
+    // 580 -> 440 us (24 rows 541, 12 rows 486). From 4,096 blocks, two such rounds, up: 2,500 parents of 4 x 25 take 113
+    // with four waves and 120 with two
+    int BT = 256;
+    if (CB * Ko <= 128 && G >= 4096 && R > 64 / CB && 64 / CB >= 8 && !getenv("FSH_FUSED_LDS_KB")) {
+        BT = 128;
+        R = 64 / CB;
+        lds = 8 * ((size_t)fused_row(K, Dk) + (size_t)CB * (Ko | 1)) * R;
+    }
+    const dim3 grid((unsigned)G), block(BT);
     // the forms with both factors fixed where they cover the pair (FSH_FUSED_FIXED=0: the run-time form, for A/B)
     const char* fxe = getenv("FSH_FUSED_FIXED");
     if (!(fxe && atoi(fxe) == 0) && (Dk == 2 || Dk == 3) && (Dp == 2 || Dp == 3)) {
         auto f = Dk == 2 ? (Dp == 2 ? launch_level_fused_k2p2 : launch_level_fused_k2p3)
                          : (Dp == 2 ? launch_level_fused_k3p2 : launch_level_fused_k3p3);
-        return f(grid, lds, s, NWK, NWP, x, P, K, c0, sl, C, hk_t, plk, Ko, hp_t, plp, Po, kc, Np, CB, R, z);
+        return f(grid, block, lds, s, NWK, NWP, x, P, K, c0, sl, C, hk_t, plk, Ko, hp_t, plp, Po, kc, Np, CB, R, z);
     }
 #define FSH_LF(A, B) hipLaunchKernelGGL((k_level_fused<A, B>), grid, block, lds, s, x, P, K, c0, sl, C, hk_t, Dk, plk, Ko, \
                                         hp_t, Dp, plp, Po, kc, Np, CB, R, z)

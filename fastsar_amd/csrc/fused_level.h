@@ -52,9 +52,9 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
     const int pad = (DK ? DK : Dk) - 1, KS = fused_row(K, DK ? DK : Dk), KoS = Ko | 1;
     float2* xs = lds_f2;                       // [R][KS]
     float2* ys = xs + (size_t)R * KS;          // [cn][R][KoS]
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, BT = blockDim.x;
     const float2* xn = x + (size_t)n * P * K;
-    for (int i = tid; i < R * 2 * pad; i += 256) {
+    for (int i = tid; i < R * 2 * pad; i += BT) {
         const int r = i / (2 * pad), e = i - r * 2 * pad;
         xs[r * KS + (e < pad ? e : K + e)] = make_float2(0.f, 0.f);
     }
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
         const float2* src = xn + (size_t)p0 * K;
         const int cnt = min(R, P - p0) * K;
         #pragma unroll
-        for (int k = 0; k < XPF; ++k) xpf[k] = load_ahead(src + min(tid + 256 * k, cnt - 1));
+        for (int k = 0; k < XPF; ++k) xpf[k] = load_ahead(src + min(tid + BT * k, cnt - 1));
     };
     prefetch(0);
     for (int p0 = 0; p0 < P; p0 += R) {
@@ -98,13 +98,13 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
             const int cnt = rn * K;
             #pragma unroll
             for (int k = 0; k < XPF; ++k) {
-                const int i = tid + 256 * k;
+                const int i = tid + BT * k;
                 if (i < cnt) {
                     const int r = i / K;
                     xs[r * KS + pad + (i - r * K)] = xpf[k];
                 }
             }
-            for (int i = tid + 256 * XPF; i < cnt; i += 256) {
+            for (int i = tid + BT * XPF; i < cnt; i += BT) {
                 const int r = i / K;
                 xs[r * KS + pad + (i - r * K)] = src[i];
             }
