@@ -10,11 +10,12 @@
 // Work: block (row p, parent n, N-group and M-chunk), four waves. The row's window goes to LDS as D planes (plane ph
 // holds x[D m + ph - pl], m = 0, 1, ...): the operand of output j at tap D u + ph is word j + u of plane ph, planes 16
 // mod 32 samples apart, so a wave's read (16 outputs, two planes, two components) falls on 64 different banks. The
-// children's taps go to LDS once a block, [child][ph][u], each (child, phase) run of ceil(L / D) taps stepped in float32
-// from a float64 seed; a lane reads the component its row and index need and flips its sign for (Re, Im x). Wave w takes
-// N-tile (8 children) w mod NTG and runs up to four M-tiles (16 outputs) a time against them, a step's operands read
-// ahead of the step before. Result: lane (output j = lane % 16, q = lane / 16) holds (Re, Im) of children 2 q and 2 q +
-// 1, rotated by rho from float64 and stored, 16 consecutive outputs of a child a time.
+// children's taps go to LDS once a block, [child][ph][u], each tap's phasor from float64 (runs of a phase's taps stepped in
+// float32 from one seed took as long, 256 us of the image below for 251, and their steps' rounding adds up: 141 taps at D 9
+// -128.2 dB from float64 against the VALU form's -130.6, -131.2 so); a lane reads the component its row and index need and
+// flips its sign for (Re, Im x). Wave w takes N-tile (8 children) w mod NTG and runs up to four M-tiles (16 outputs) a time
+// against them, a step's operands read ahead of the step before. Result: lane (output j = lane % 16, q = lane / 16) holds
+// (Re, Im) of children 2 q and 2 q + 1, rotated by rho from float64 and stored, 16 consecutive outputs of a child a time.
 //
 // Bound by the float32 matrix rate (the VALU's; no operand is rounded) and, at two waves a SIMD, by the reads of a step.
 // 534 x 534 image from 1,400 x 4,088 samples (D 16, 134 taps, 25 children): 1,395 us on the VALU kernel, which read two
@@ -77,24 +78,21 @@ __global__ __launch_bounds__(256) void k_rot_fir_k_f32(const float2* __restrict_
         if (D2 > D)                                        // an odd count of phases: a plane of zeros
             for (int i = tid; i < WM; i += 256) X[(size_t)D * PS + i] = make_float2(0.f, 0.f);
     }
-    // taps: run (child, ph): exp(2 pi i sl ph) in float64, then steps of exp(2 pi i sl D)
+    // taps: run (child, ph), every tap's phasor from float64
     for (int e = tid; e < 8 * NTG * D2; e += 256) {
         const int c = e / D2, ph = e - c * D2;
         float2* g = reinterpret_cast<float2*>(G + (size_t)c * CS) + ph * Up;
         const bool ok = cb + c < Cn && ph < D;
-        float cs = 0.f, sn = 0.f, dc = 0.f, dn = 0.f;
-        if (ok) {
-            const double b = (double)sl[((size_t)n * Cn + cb + c) * P + p];
-            cis_cyc((double)ph * b, cs, sn);
-            cis_cyc((double)D * b, dc, dn);
-        }
+        const double b = ok ? (double)sl[((size_t)n * Cn + cb + c) * P + p] : 0.0;
         for (int u = 0; u < U; ++u) {
             const int r = D * u + ph;
-            const float h = ok && r < L ? taps[r] : 0.f;
-            g[u] = make_float2(h * cs, h * sn);
-            const float nc = fmaf(cs, dc, -(sn * dn));
-            sn = fmaf(cs, dn, sn * dc);
-            cs = nc;
+            float2 v = make_float2(0.f, 0.f);
+            if (ok && r < L) {
+                float cs, sn;
+                cis_cyc((double)r * b, cs, sn);
+                v = make_float2(taps[r] * cs, taps[r] * sn);
+            }
+            g[u] = v;
         }
     }
     __syncthreads();
@@ -153,7 +151,7 @@ __global__ __launch_bounds__(256) void k_rot_fir_k_f32(const float2* __restrict_
 }
 
 // the launch's shape: as many N-tiles a block as its waves (four) and as few M-chunks as fit 80 KB of LDS (two blocks a
-// CU), else 156 KB; false where not even one N-tile and M-tile fit, or a run of taps is longer than 16 float32 steps
+// CU), else 156 KB; false where not even one N-tile and M-tile fit, or a phase has more than 16 taps
 static bool f32_shape(int L, int D, int Ko, int Cn, F32Shape& s)
 {
     if (D < 2) return false;
