@@ -19,7 +19,8 @@
 //
 // Bound by the float32 matrix rate (the VALU's; no operand is rounded) and, at two waves a SIMD, by the reads of a step.
 // 534 x 534 image from 1,400 x 4,088 samples (D 16, 134 taps, 25 children): 1,395 us on the VALU kernel, which read two
-// LDS words a tap and output, 262 us here (10 GFLOP of real products, 38 TFLOP/s).
+// LDS words a tap and output, 257 us here (10 GFLOP of real products, 39 TFLOP/s). Two waves a SIMD are all that LDS leaves,
+// and declared, so that the sums stay in VGPRs: in AGPRs the compiler moved 12 of them a step (262 us).
 #include "fsh_common.h"
 #include "fsh_kernels.h"
 
@@ -31,6 +32,12 @@ namespace {
 
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
+// Contraction steps of one chain of sums (four products each); the chains' results are added. One chain of all 2 L products
+// rounds above the VALU form, which deals an output's taps to several threads where a block has few outputs: -127.8 dB from
+// float64 against -130.2 at 261 taps, -134.2 in chains of 32 steps, -136.5 of 11. First level of the 534 x 534 image above:
+// 251 us in one chain, 257 in chains of 32 steps, 255 of 64.
+constexpr int SUM_STEPS = 32;
+
 struct F32Shape {
     int U, Up, D2, CS, PS, NTG, MC, chunks, ngroups;
     size_t lds;
@@ -38,10 +45,11 @@ struct F32Shape {
 
 }  // namespace
 
-__global__ __launch_bounds__(256) void k_rot_fir_k_f32(const float2* __restrict__ x, int P, int K, const float* __restrict__ c0,
-                                                       const float* __restrict__ sl, int Cn, const float* __restrict__ taps,
-                                                       int L, int pl, int D, int Ko, double kc, int U, int Up, int D2, int CS,
-                                                       int PS, int NTG, int MC, int chunks, float2* __restrict__ y)
+__global__ __launch_bounds__(256, 2) void k_rot_fir_k_f32(const float2* __restrict__ x, int P, int K,
+                                                          const float* __restrict__ c0, const float* __restrict__ sl, int Cn,
+                                                          const float* __restrict__ taps, int L, int pl, int D, int Ko,
+                                                          double kc, int U, int Up, int D2, int CS, int PS, int NTG, int MC,
+                                                          int chunks, float2* __restrict__ y)
 {
     extern __shared__ float lds_f[];
     float2* X = reinterpret_cast<float2*>(lds_f);          // [D2][PS]
@@ -111,24 +119,29 @@ __global__ __launch_bounds__(256) void k_rot_fir_k_f32(const float2* __restrict_
         #pragma unroll
         for (int m = 0; m < 4; ++m) off[m] = 32 * min(m, m1 - 1 - mg);
         int u = 0, go = 0, xo = 0;                         // offsets (floats) of the step to read next
-        auto advance = [&]() {
-            ++u; go += 2; xo += 2;
-            if (u == U) { u = 0; go += 4 * Up - 2 * U; xo += 4 * PS - 2 * U; }
-        };
         float gn = ga[0], xn[4];
         #pragma unroll
         for (int m = 0; m < 4; ++m) xn[m] = xm[off[m]];
-        for (int s = 0; s < steps; ++s) {
-            const float g = __uint_as_float(__float_as_uint(gn) ^ flip);
-            float xv[4];
+        for (int s0 = 0; s0 < steps; s0 += SUM_STEPS) {
+            floatx4_t part[4] = {};
+            for (int s = s0; s < min(s0 + SUM_STEPS, steps); ++s) {
+                const float g = __uint_as_float(__float_as_uint(gn) ^ flip);
+                float xv[4];
+                #pragma unroll
+                for (int m = 0; m < 4; ++m) xv[m] = xn[m];
+                const bool wrap = ++u == U;
+                go += wrap ? 4 * Up - 2 * U + 2 : 2;
+                xo += wrap ? 4 * PS - 2 * U + 2 : 2;
+                u = wrap ? 0 : u;
+                if (s + 1 == steps) go = xo = 0;           // (read, not used)
+                gn = ga[go];
+                #pragma unroll
+                for (int m = 0; m < 4; ++m) xn[m] = xm[xo + off[m]];
+                #pragma unroll
+                for (int m = 0; m < 4; ++m) part[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, xv[m], part[m], 0, 0, 0);
+            }
             #pragma unroll
-            for (int m = 0; m < 4; ++m) xv[m] = xn[m];
-            if (s + 1 < steps) advance();                  // the last step reads its own operands again
-            gn = ga[go];
-            #pragma unroll
-            for (int m = 0; m < 4; ++m) xn[m] = xm[xo + off[m]];
-            #pragma unroll
-            for (int m = 0; m < 4; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, xv[m], acc[m], 0, 0, 0);
+            for (int m = 0; m < 4; ++m) acc[m] += part[m];
         }
         #pragma unroll
         for (int e = 0; e < 2; ++e) {

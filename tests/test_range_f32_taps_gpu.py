@@ -1,7 +1,7 @@
-"""The float32 matrix range filter's complex taps: its error against float64 may not pass that of the VALU form
-(FSH_ROT_KERNEL=valu), which seeds runs of five to seven taps in float64, on the same inputs. Both sum an output's 2 L
-products in float32 chains of the same length, so a larger error can only come from the taps' phasors. The phase slopes
-reach 0.8 cycles a sample and the filters have 9 to 16 taps a phase, 16 being the most the form takes.
+"""The float32 matrix range filter's complex taps and sums: its error against float64 may not pass that of the VALU form
+(FSH_ROT_KERNEL=valu) on the same inputs, which seeds runs of four to eight taps in float64 and, where a row's window leaves
+a block few outputs, deals an output's taps to several threads. The phase slopes reach 0.8 cycles a sample; the filters
+have 134 to 434 taps, 7 to 16 a phase, 16 being the most the form takes.
 
 0.1 dB is allowed for the two orders of the sums: the mean square of the error over n outputs scatters by sqrt(2 / n),
 0.04 dB at 20,000 outputs, so 0.06 dB for the ratio of two."""
@@ -14,7 +14,8 @@ from oracle import plain_db as db
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(16, 0.47, 25, 1100), (12, 0.66, 32, 900), (9, 0.72, 25, 1300)]
+CASES = [(16, 0.47, 25, 1100), (12, 0.66, 32, 900), (9, 0.72, 25, 1300), (25, 0.58, 16, 2400),
+         (25, 0.36, 17, 2400), (30, 0.7, 16, 2700), (40, 0.6, 19, 3200)]
 
 
 @pytest.mark.parametrize('D,pf,Cn,K', CASES)
