@@ -1171,15 +1171,17 @@ int launch_rot_fir_k(const float2* x, int Np, int P, int K, const float* c0, con
         set_error("rot_fir_k: invalid shape");
         return E_INVALID;
     }
-    // the matrix-core form where its taps fit (L <= 128) and the axis is decimated; FSH_ROT_KERNEL=valu|mfma forces one
-    // FSH_ROT_KERNEL=valu|mfma|mfma1 forces one (mfma: the row kernel where its taps fit; mfma1: the per-wave-row
-    // form); by default the row kernel for rows of four or more M-tiles, the per-wave-row form below that
+    // the matrix-core form where its taps fit (L <= 128) and the axis is decimated.
+    // FSH_ROT_KERNEL=valu|mfma|mfma1|f32 forces one (mfma: the row kernel where its taps fit; mfma1: the per-wave-row
+    // form; f32: the float32 matrix form where it fits LDS); by default the row kernel for rows of four or more M-tiles,
+    // the per-wave-row form below that
     const char* force = getenv("FSH_ROT_KERNEL");
     const bool want_long = force && strcmp(force, "long") == 0;
     const bool want_valu = (force && strcmp(force, "valu") == 0) || want_long;
+    const bool want_f32 = force && strcmp(force, "f32") == 0;
     const bool want_mfma1 = force && strcmp(force, "mfma1") == 0;
     const bool want_mfma = (force && strcmp(force, "mfma") == 0) || want_mfma1;
-    if (!want_valu && (D > 1 || want_mfma) && L <= 128) {
+    if (!want_valu && !want_f32 && (D > 1 || want_mfma) && L <= 128) {
         int st = E_INVALID;
         // the row form amortizes each row's taps over its M-tiles: it wins from four M-tiles (128 outputs) up
         const bool row_form = force && strcmp(force, "mfma") == 0 ? true : (Ko + 31) / 32 >= 4;
@@ -1191,17 +1193,23 @@ int launch_rot_fir_k(const float2* x, int Np, int P, int K, const float* c0, con
         if (st == E_INVALID) st = launch_rot_fir_k_mfma(x, Np, P, K, c0, sl, Cn, taps, L, pl, D, Ko, kc, y, s);
         if (st != E_INVALID) return st;
     }
-    // longer filters on the float32 matrix instructions where their window and taps fit LDS
-    if (!force && D > 1) {
-        const int st = launch_rot_fir_k_f32(x, Np, P, K, c0, sl, Cn, taps, L, pl, D, Ko, kc, y, s);
-        if (st != E_INVALID) return st;
-    }
     const int PB = 8;
     const int budget = std::min(lds_limit(), 65536);
     int JB = 64;
     auto need = [&](int jb) { const int W = D * (jb - 1) + L; return PB * (W + L) * 8; };
     while (JB > 4 && need(JB) > budget) JB /= 2;
-    if (need(JB) > budget || want_long) {
+    const bool window_fits = need(JB) <= budget;
+    // Longer filters on the float32 matrix instructions, in place of the VALU form (k_rot_fir_k), where the children fill
+    // enough of a block's eight slots: it builds a row's taps for all eight, which grows with D, and saves time a child.
+    // 1,000 rows, VALU -> matrix: 25 children at D 16 (176 taps) 2,175 -> 349 us, 9 at D 30 (326) 672 -> 244, 4 at D 16
+    // 155 -> 36, 4 at D 40 (318) 254 -> 152; past the line 4 at D 64 (398) 59 -> 73, 3 at D 55 (343) 44 -> 66, 2 at D 40
+    // (434) 45 -> 70. Never in place of k_rot_fir_k_long, whose 64 lanes an output add shorter chains (D 64, 556 taps: -137.1
+    // dB from float64 for -133.8) and which is the faster at large D (D 120, 1,298 taps, 9 children: 484 us for 1,314).
+    if (want_f32 || (!force && D > 1 && window_fits && D <= 16 * Cn - 24)) {
+        const int st = launch_rot_fir_k_f32(x, Np, P, K, c0, sl, Cn, taps, L, pl, D, Ko, kc, y, s);
+        if (st != E_INVALID) return st;
+    }
+    if (!window_fits || want_long) {
         // a window longer than any LDS tile: the direct form (FSH_ROT_KERNEL=long forces it, for tests)
         const int JW = 16;
         for (int n0 = 0; n0 < Np; n0 += 65535) {
