@@ -723,7 +723,7 @@ int fsh_ffbp_create(const fsh_plan_desc* plan, const fsh_level_desc* levels, voi
             // later levels take a one-pass form where one applies (level 0's children come in groups): on VALU for
             // short children whose parent one block holds, else on the matrix cores, else the two-pass form
             const int Lk = h.Dk > 1 ? h.Lk : 1, Lp = h.Dp > 1 ? h.Lp : 1;
-            if (l > 0 && level_fused_preferred(h.C, h.P, h.K, Lk, h.Dk, h.Ko, Lp, h.Dp)) {
+            if (l > 0 && level_fused_preferred(h.nparents, h.C, h.P, h.K, Lk, h.Dk, h.Ko, Lp, h.Dp)) {
                 f->const_bytes += ((size_t)h.Dk * fused_nw(Lk, h.Dk) + (size_t)h.Dp * fused_nw(Lp, h.Dp)) * sizeof(float);
                 if ((st = dev_alloc((void**)&L.hk_t, (size_t)h.Dk * fused_nw(Lk, h.Dk) * sizeof(float))) ||
                     (st = dev_alloc((void**)&L.hp_t, (size_t)h.Dp * fused_nw(Lp, h.Dp) * sizeof(float))) ||

@@ -53,7 +53,7 @@ bool fir_p_streams(int L, int D);
 // polyphase tables that launch_polyphase builds from the taps (h == nullptr: the unit tap of an undecimated axis)
 int fused_nw(int L, int D);
 bool level_fused_shape(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int Dp, int& CB, int& R, size_t& lds);
-bool level_fused_preferred(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int Dp);
+bool level_fused_preferred(long parents, int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int Dp);
 int launch_polyphase(const float* h, int L, int D, float* t, hipStream_t s);
 int launch_polyphase_nw(const float* h, int L, int D, int NW, float* t, hipStream_t s);
 // a level on the matrix cores with the pulse filter fused (level_mfma.hip): both axes decimated, hp_t the pulse

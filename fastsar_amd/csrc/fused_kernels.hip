@@ -95,9 +95,13 @@ bool level_fused_shape(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int 
 // parent's rows are read once) and they cover a quarter of its threads or more; the other forms where the children are
 // long or many. From 64 columns, not 128: a 2048 x 2048 image's level 3 (16,384 parents of 4 x 29 columns) takes 440 us
 // here and 1,200 on the one-pass matrix-core form, whose blocks of 8 children it half fills (and in float32, where that
-// form's range products are bfloat16 x 3). FSH_LEVEL_KERNEL=fused forces it where it applies, =split or =mfma turns it
-// off.
-bool level_fused_preferred(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int Dp)
+// form's range products are bfloat16 x 3). That form takes both axes decimated; with either left alone the other is the
+// two-pass form, whose time goes with the children and this one's, a block a parent, with the pulses until the blocks
+// fill the device, so that 64 to 127 columns come here from 1,024 children on, or where a pulse filter would walk 80 rows
+// or fewer. Range alone decimated, 4 children a parent, 200 pulses: 64 parents 64 us here for 21, 128 65 for 39, 256 67
+// for 75, 1,024 152 for 288; pulses alone: 64 parents of 200 rows 61 for 37, of 60 rows 19 for 26. FSH_LEVEL_KERNEL=fused
+// forces it where it applies, =split or =mfma turns it off.
+bool level_fused_preferred(long parents, int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int Dp)
 {
     int CB, R;
     size_t lds;
@@ -105,7 +109,8 @@ bool level_fused_preferred(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, 
     const char* force = getenv("FSH_LEVEL_KERNEL");
     if (force && strcmp(force, "fused") == 0) return true;
     if (force && strcmp(force, "mfma") == 0) return false;
-    return CB == C && CB * Ko >= 64;
+    if (CB < C || C * Ko < 64) return false;
+    return C * Ko >= 128 || (Dk > 1 && Dp > 1) || parents * C >= 1024 || (Dp > 1 && P <= 80);
 }
 
 int launch_level_fused(const float2* x, int Np, int P, int K, const float* c0, const float* sl, int C, const float* hk_t,
