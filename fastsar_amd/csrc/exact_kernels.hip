@@ -469,7 +469,7 @@ struct Exact {
     double* ramp = nullptr;          // [P] (a, b) cycles: the phase re-reference applied on the way in (fsh_exact_set_ramp)
     bool use_ramp = false;
     float2* image = nullptr;         // [nseg, nx, ny]
-    int nseg = 1;                    // images the pulses of each chunk are dealt to (bp_segments)
+    int seg = 1, nseg = 1;           // pulses a workgroup takes of a chunk (bp_share), images they are dealt to
     int* bad = nullptr;
     int* bad_host = nullptr;         // its value after a call (pinned)
     hipfftHandle plan = 0;
@@ -546,15 +546,17 @@ static bool bp_shape(const fsh_exact_desc& d, BpShape& sh)
     return false;
 }
 
-// Images the pulses of a chunk are dealt to: a grid of few regions (1,024 pixels a workgroup, five workgroups a CU, each
-// one serial in its pulses) would leave the device idle, so that many workgroups share a region, up to 16, with 64
-// pulses or more each; their images are added at the end. From 641 regions up one image: two workgroups a region of
-// 1,024 regions would run in two rounds for one. 113 x 2,179 pixels (276 regions) from 1,916 pulses 2,400 -> 650 us, 121 x
-// 652 (84) from 628 1,398 -> 278, 1,568 x 261 (441) from 743 703 -> 474
-static int bp_segments(const fsh_exact_desc& d, int BR)
+// Pulses of a chunk that a workgroup takes: a grid of few regions (1,024 pixels a workgroup, five workgroups a CU, each
+// one serial in its pulses) would leave the device idle, so that up to 16 workgroups share a region, with 64 pulses or more
+// each, in whole batches of NB; each adds into an image of its own, the images are added at the end. From 641 regions up
+// one image: two workgroups a region of 1,024 regions would run in two rounds for one. 113 x 2,179 pixels (276 regions)
+// from 1,916 pulses 2,400 -> 650 us, 121 x 652 (84) from 628 1,398 -> 278, 1,568 x 261 (441) from 743 703 -> 474
+static int bp_share(const fsh_exact_desc& d, const BpShape& sh)
 {
-    const long G = (long)((d.nx + BR - 1) / BR) * ((d.ny + BR - 1) / BR);
-    return (int)std::max<long>(1, std::min<long>(std::min<long>(16, 1280 / G), std::min(d.chunk, d.P) / 64));
+    const long G = (long)((d.nx + sh.BR - 1) / sh.BR) * ((d.ny + sh.BR - 1) / sh.BR);
+    const int ch = std::min(d.chunk, d.P);
+    const int n = (int)std::max<long>(1, std::min<long>(std::min<long>(16, 1280 / G), ch / 64));
+    return n == 1 ? ch : (ch + n * sh.NB - 1) / (n * sh.NB) * sh.NB;
 }
 
 template <int BR, int TX, int TY, int PT>
@@ -594,7 +596,7 @@ static int launch_bp(const Exact& e, int n, int p0, float2* out)
     a.win = d.profiles ? e.winh : (const void*)e.win;
     a.smax = e.smax;
     a.P = n;
-    a.seg = e.nseg > 1 ? (std::min(d.chunk, d.P) + e.nseg * sh.NB - 1) / (e.nseg * sh.NB) * sh.NB : n;   // whole batches
+    a.seg = e.seg;
     a.W = d.W;
     a.nfft = d.nfft;
     a.NB = sh.NB;
@@ -658,7 +660,9 @@ int fsh_exact_create(const fsh_exact_desc* desc, void** handle)
     }
     Exact* e = new Exact();
     e->d = d;
-    e->nseg = bp_segments(d, sh.BR);
+    const int ch = std::min(d.chunk, d.P);
+    e->seg = bp_share(d, sh);
+    e->nseg = (ch + e->seg - 1) / e->seg;
     {
         // the line of sight from the track's mean to the grid's mean, against the grid's axes: the axis it has the
         // smaller part along is the across-range one
@@ -682,7 +686,6 @@ int fsh_exact_create(const fsh_exact_desc* desc, void** handle)
     e->d.ant = e->d.ref = e->d.cen = nullptr;
     e->d.blo = nullptr;
     e->d.wp = e->d.wk = nullptr;
-    const int ch = std::min(d.chunk, d.P);
     if ((st = dev_alloc((void**)&e->pad, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->prof, (size_t)ch * d.nfft * sizeof(float2))) ||
         (st = dev_alloc((void**)&e->win, (size_t)ch * d.W * sizeof(float2))) ||
@@ -690,6 +693,7 @@ int fsh_exact_create(const fsh_exact_desc* desc, void** handle)
         return fail(st);
     st = dev_alloc((void**)&e->image, (size_t)e->nseg * d.nx * d.ny * sizeof(float2));
     if (st == E_NOMEM && e->nseg > 1) {                    // one image where several do not fit
+        e->seg = ch;
         e->nseg = 1;
         st = dev_alloc((void**)&e->image, (size_t)d.nx * d.ny * sizeof(float2));
     }
