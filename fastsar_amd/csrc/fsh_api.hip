@@ -593,7 +593,7 @@ int fsh_level_mfma(const float* x, int Np, int P, int K, const float* c0, const 
     if (!x || !c0 || !sl || !z || !taps_k || !taps_p) { set_error("level_mfma: null argument"); return E_INVALID; }
     int KS, NWp, NPH, PS, JT, njr, nseg, IS, nwp, tpw, nwv;
     size_t lds;
-    if (Np < 1 || Lk < 1 || Lp < 1 || !level_mfma_shape(Np, Cn, Lk, Dk, Ko, Lp, Dp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS,
+    if (Np < 1 || P < 1 || Lk < 1 || Lp < 1 || plp < 0 || !level_mfma_shape(Np, P, Cn, Lk, Dk, Ko, Lp, Dp, plp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS,
                                                         lds, nwp, tpw, nwv)) {
         set_error("level_mfma: the level does not fit the fused matrix-core form (Dk, Dp >= 2, Ko >= 16, Dk ceil(Lk / Dk) "
                   "<= 128, ceil(Lp / Dp) <= 16)");
@@ -620,7 +620,7 @@ int fsh_level_mfma_noalloc(const float* x, int Np, int P, int K, const float* c0
     if (!x || !c0 || !sl || !z || !taps_k || !taps_p) { set_error("level_mfma_noalloc: null argument"); return E_INVALID; }
     int KS, NWp, NPH, PS, JT, njr, nseg, IS, nwp, tpw, nwv;
     size_t lds;
-    if (Np < 1 || Lk < 1 || Lp < 1 || !level_mfma_shape(Np, Cn, Lk, Dk, Ko, Lp, Dp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS,
+    if (Np < 1 || P < 1 || Lk < 1 || Lp < 1 || plp < 0 || !level_mfma_shape(Np, P, Cn, Lk, Dk, Ko, Lp, Dp, plp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS,
                                                         lds, nwp, tpw, nwv)) {
         set_error("level_mfma_noalloc: the level does not fit the fused matrix-core form (Dk, Dp >= 2, Ko >= 16, "
                   "Dk ceil(Lk / Dk) <= 128, ceil(Lp / Dp) <= 16)");
@@ -643,6 +643,20 @@ int fsh_level_mfma_noalloc(const float* x, int Np, int P, int K, const float* c0
         if (e != hipSuccess) st = hip_status(e, "level_mfma_noalloc");
     }
     return st;
+}
+
+int fsh_level_mfma_segments(int Np, int P, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int plp, int Po, int* segments)
+{
+    if (!segments) { set_error("level_mfma_segments: null argument"); return E_INVALID; }
+    int KS, NWp, NPH, PS, JT, njr, nseg, IS, nwp, tpw, nwv;
+    size_t lds;
+    if (Np < 1 || P < 1 || Lk < 1 || Lp < 1 || Po < 1 || plp < 0 ||
+        !level_mfma_shape(Np, P, C, Lk, Dk, Ko, Lp, Dp, plp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS, lds, nwp, tpw, nwv)) {
+        set_error("level_mfma_segments: the level does not fit the fused matrix-core form");
+        return E_INVALID;
+    }
+    *segments = nseg;
+    return OK;
 }
 
 int fsh_device_phases(const double* refs, const double* u, const double* r0, const double* d, int Np, int Cn, int P,

@@ -59,8 +59,8 @@ int launch_polyphase_nw(const float* h, int L, int D, int NW, float* t, hipStrea
 // a level on the matrix cores with the pulse filter fused (level_mfma.hip): both axes decimated, hp_t the pulse
 // filter's polyphase table for level_mfma_nw(Lp, Dp) accumulators
 int level_mfma_nw(int Lp, int Dp);
-bool level_mfma_shape(int Np, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int Po, int& KS, int& NWp, int& NPH, int& PS,
-                      int& JT, int& njr, int& nseg, int& IS, size_t& lds, int& nwp, int& tpw, int& nwv);
+bool level_mfma_shape(int Np, int P, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int plp, int Po, int& KS, int& NWp,
+                      int& NPH, int& PS, int& JT, int& njr, int& nseg, int& IS, size_t& lds, int& nwp, int& tpw, int& nwv);
 bool level_mfma_preferred(int C, int Lk, int Dk, int Ko, int Lp, int Dp, int Po);
 bool level_mfma_split_input(int C, int Lk, int Dk, int Ko, int Lp, int Dp, int Po);
 // xsplit: x holds each sample as its bfloat16 x 3 words (hi, lo) (launch_fir_p with split), staged without a split

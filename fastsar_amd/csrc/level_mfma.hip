@@ -421,8 +421,8 @@ int level_mfma_nw(int Lp, int Dp)
     return -1;
 }
 
-bool level_mfma_shape(int Np, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int Po, int& KS, int& NWp, int& NPH, int& PS,
-                      int& JT, int& njr, int& nseg, int& IS, size_t& lds, int& nwp, int& tpw, int& nwv)
+bool level_mfma_shape(int Np, int P, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int plp, int Po, int& KS, int& NWp,
+                      int& NPH, int& PS, int& JT, int& njr, int& nseg, int& IS, size_t& lds, int& nwp, int& tpw, int& nwv)
 {
     if (Dk < 2 || Dp < 2 || C < 1 || Ko < 16) return false;
     const int NW = (Lk + Dk - 1) / Dk;
@@ -468,20 +468,34 @@ bool level_mfma_shape(int Np, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int
     if (Dk * (16 * JT + NWp) > maxi * nthr || Dk * NWp > TAB_MAX || CB * NE > ef_items(tpw) * nthr ||
         CB * (4 * JT + 1) > (tpw == 1 ? 1 : 2) * nthr)
         return false;
-    // segments of output pulses, each re-reading Lp rows: the count with the least time by a model of the walk. A CU holds
-    // `occ` blocks (LDS, four waves a SIMD); k blocks on it take 1 + 0.06 (k - 1) nwv times one block's time a row (a
-    // barrier a row: measured 1.35-1.48 for two blocks of 6 or 7 waves, 1.43 from two to four of 4, 1.18 of 3), and a
-    // block's start about 12 rows' time. The halving rule before (2,048 blocks, a halo below a fifth) left images of few
-    // parents on a quarter of the CUs: 64 parents of 4 children, 266 rows 181 -> 100 us (8 segments for 1), 25 of 9, 477
-    // rows 355 -> 164, 16 of 4, 190 rows 125 -> 40; and cut past a whole round: 56 of 48, 2,058 rows 3.26 -> 3.02 ms
+    // segments of output pulses, each re-reading Lp rows of those there are: the count with the least time by a model of the
+    // walk. A CU holds `occ` blocks (LDS, four waves a SIMD); k blocks on it take 1 + 0.06 (k - 1) nwv times one block's
+    // time a row (a barrier a row: measured 1.35-1.48 for two blocks of 6 or 7 waves, 1.43 from two to four of 4, 1.18 of
+    // 3), and a block's start about 12 rows' time. The halving rule before (2,048 blocks, a halo below a fifth) left images
+    // of few parents on a quarter of the CUs: 64 parents of 4 children, 266 rows 181 -> 100 us (8 segments for 1), 25 of 9,
+    // 477 rows 355 -> 164, 16 of 4, 190 rows 125 -> 40; and cut past a whole round: 56 of 48, 2,058 rows 3.26 -> 3.02 ms.
+    // Rows off the axis are not walked and not counted: with them, 144 parents of 4 x 99 columns, 60 rows took three
+    // segments, the longest of 58 rows, and 172 us for 95.
     const int occ = std::max(1, std::min((int)(160 * 1024 / lds), 16 / nwv));
     auto load = [&](long k) { return k ? 1.0 + 0.06 * (k - 1) * nwv : 0.0; };
+    // rows that the longest of the segments of `is` outputs walks: the first whose rows begin inside the axis, or the one
+    // before it
+    auto rows = [&](int is, int ns) {
+        int most = 1;
+        const int s1 = (plp + Dp * is - 1) / (Dp * is);
+        for (int sg = std::max(0, s1 - 1); sg <= std::min(s1, ns - 1); ++sg) {
+            const long i0 = (long)sg * is, i1 = std::min((long)Po, i0 + is);
+            most = (int)std::max<long>(most, std::min<long>(P, Dp * (i1 - 1) - plp + Lp) - std::max<long>(0, Dp * i0 - plp));
+        }
+        return most;
+    };
+    const long blocks0 = (long)Np * ((C + CB - 1) / CB) * njr;
     double best = 0.0;
     IS = 0;
     for (int n = 1; n <= std::min(Po, 64); ++n) {
         const int is = (Po + n - 1) / n, ns = (Po + is - 1) / is;
-        const long k = ((long)Np * ((C + CB - 1) / CB) * njr * ns + 255) / 256;
-        const double t = ((k / occ) * load(occ) + load(k % occ)) * ((double)Dp * is + Lp + 12);
+        const long k = (blocks0 * ns + 255) / 256;
+        const double t = ((k / occ) * load(occ) + load(k % occ)) * (rows(is, ns) + 12);
         if (!IS || t < best) { best = t; IS = is; nseg = ns; }
     }
     return true;
@@ -497,7 +511,7 @@ bool level_mfma_preferred(int C, int Lk, int Dk, int Ko, int Lp, int Dp, int Po)
     if (force && (strcmp(force, "split") == 0 || strcmp(force, "fused") == 0)) return false;
     int KS, NWp, NPH, PS, JT, njr, nseg, IS, nwp, tpw, nwv;
     size_t lds;
-    if (!level_mfma_shape(1, C, Lk, Dk, Ko, Lp, Dp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS, lds, nwp, tpw, nwv)) return false;
+    if (!level_mfma_shape(1, Po, C, Lk, Dk, Ko, Lp, Dp, 0, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS, lds, nwp, tpw, nwv)) return false;
     const char* rows = getenv("FSH_LMFMA_ROWS");
     return (force && strcmp(force, "mfma") == 0) || (njr == 1 && tpw == 1) || (rows && atoi(rows) == 1 && tpw == 1);
 }
@@ -507,7 +521,7 @@ bool level_mfma_split_input(int C, int Lk, int Dk, int Ko, int Lp, int Dp, int P
 {
     int KS, NWp, NPH, PS, JT, njr, nseg, IS, nwp, tpw, nwv;
     size_t lds;
-    return level_mfma_shape(1, C, Lk, Dk, Ko, Lp, Dp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS, lds, nwp, tpw, nwv) && tpw == 1;
+    return level_mfma_shape(1, Po, C, Lk, Dk, Ko, Lp, Dp, 0, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS, lds, nwp, tpw, nwv) && tpw == 1;
 }
 
 // hp_t: the pulse filter's polyphase table for level_mfma_nw(Lp, Dp) accumulators (launch_polyphase_nw)
@@ -518,7 +532,7 @@ int launch_level_mfma(const float2* x, int Np, int P, int K, const float* c0, co
     int KS, NWp, NPH, PS, JT, njr, nseg, IS, nwp, tpw, nwv;
     size_t lds;
     if (Np < 1 || P < 1 || K < 1 || plk < 0 || plp < 0 ||
-        !level_mfma_shape(Np, C, Lk, Dk, Ko, Lp, Dp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS, lds, nwp, tpw, nwv)) {
+        !level_mfma_shape(Np, P, C, Lk, Dk, Ko, Lp, Dp, plp, Po, KS, NWp, NPH, PS, JT, njr, nseg, IS, lds, nwp, tpw, nwv)) {
         set_error("level_mfma: the level does not fit the fused matrix-core form");
         return E_INVALID;
     }

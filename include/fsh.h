@@ -97,6 +97,10 @@ int fsh_level_mfma_noalloc(const float* x, int Np, int P, int K, const float* c0
                            const float* taps_k, int Lk, int plk, int Dk, int Ko, const float* taps_p, int Lp, int plp, int Dp,
                            int Po, double kc, float* z, void* stream);
 
+/* The segments of output pulses that fsh_level_mfma cuts a level's walk along the pulses into (host only; FSH_EINVAL where
+ * the level does not fit). Results do not depend on it. No counterpart in the reference: for tests and measurements. */
+int fsh_level_mfma_segments(int Np, int P, int Cn, int Lk, int Dk, int Ko, int Lp, int Dp, int plp, int Po, int* segments);
+
 /* Child rotations of a level computed on the device in float64: refs [Np, 3] parent centres, u [P, 3], r0 [P] the
  * level's track, d [Cn, 3] child offsets -> c0, sl [Np, Cn, P] float32. Replaces the device-phase kernel and the
  * host form (fastsar/ffbp_cuda.py:598-632, fastsar/ffbp_cpu.py:142-155). */
