@@ -469,15 +469,19 @@ bool level_mfma_shape(int Np, int P, int C, int Lk, int Dk, int Ko, int Lp, int 
         CB * (4 * JT + 1) > (tpw == 1 ? 1 : 2) * nthr)
         return false;
     // segments of output pulses, each re-reading Lp rows of those there are: the count with the least time by a model of the
-    // walk. A CU holds `occ` blocks (LDS, four waves a SIMD); k blocks on it take 1 + 0.06 (k - 1) nwv times one block's
-    // time a row (a barrier a row: measured 1.35-1.48 for two blocks of 6 or 7 waves, 1.43 from two to four of 4, 1.18 of
-    // 3), and a block's start about 12 rows' time. The halving rule before (2,048 blocks, a halo below a fifth) left images
-    // of few parents on a quarter of the CUs: 64 parents of 4 children, 266 rows 181 -> 100 us (8 segments for 1), 25 of 9,
-    // 477 rows 355 -> 164, 16 of 4, 190 rows 125 -> 40; and cut past a whole round: 56 of 48, 2,058 rows 3.26 -> 3.02 ms.
-    // Rows off the axis are not walked and not counted: with them, 144 parents of 4 x 99 columns, 60 rows took three
-    // segments, the longest of 58 rows, and 172 us for 95.
-    const int occ = std::max(1, std::min((int)(160 * 1024 / lds), 16 / nwv));
-    auto load = [&](long k) { return k ? 1.0 + 0.06 * (k - 1) * nwv : 0.0; };
+    // walk. A CU holds `occ` blocks: LDS, and four waves a SIMD (128 registers; three past 10 accumulators a filter), of
+    // which a block of more than four waves takes its fullest SIMD's count on each. k blocks on it take 1 + 0.05 (k - 1)
+    // nwv times one block's time a row (measured beside a lone block: 1.10 for two of 5 waves, 1.18 of 7, 1.15 for four of
+    // 3, 1.33 five), and a block's start about 4 rows' time. Against the best of nine counts at 1,148 shapes (4 to 16
+    // children, 20 to 150 columns, 60 to 900 rows, 4 to 900 parents) 0.8 % more time, 24 % at the worst. The halving rule
+    // before (2,048 blocks, a halo below a fifth) took 1.55 times as long over 3,390 such shapes: 64 parents of 4 children,
+    // 266 rows 181 us for 100, 25 of 9, 477 rows 355 for 164, 16 of 4, 190 rows 125 for 40. Rows off the axis are not walked
+    // and not counted: with them, 144 parents of 4 x 99 columns, 60 rows took three segments, the longest of 58 rows, and
+    // 172 us for 95. With 16 waves' room whatever the registers, 256 parents of 4 x 66 columns, 100 rows took three
+    // segments, whose five-wave blocks of 145 registers take turns, and 248 us for 138.
+    const int slots = nwp <= 10 ? 4 : 3;
+    const int occ = std::max(1, std::min((int)(160 * 1024 / lds), nwv >= 4 ? slots / ((nwv + 3) / 4) : 4 * slots / nwv));
+    auto load = [&](long k) { return k ? 1.0 + 0.05 * (k - 1) * nwv : 0.0; };
     // rows that the longest of the segments of `is` outputs walks: the first whose rows begin inside the axis, or the one
     // before it
     auto rows = [&](int is, int ns) {
@@ -492,10 +496,10 @@ bool level_mfma_shape(int Np, int P, int C, int Lk, int Dk, int Ko, int Lp, int 
     const long blocks0 = (long)Np * ((C + CB - 1) / CB) * njr;
     double best = 0.0;
     IS = 0;
-    for (int n = 1; n <= std::min(Po, 64); ++n) {
+    for (int n = 1; n <= std::min(Po, 64); n += n < 16 ? 1 : n < 32 ? 4 : n < 48 ? 8 : 16) {
         const int is = (Po + n - 1) / n, ns = (Po + is - 1) / is;
         const long k = (blocks0 * ns + 255) / 256;
-        const double t = ((k / occ) * load(occ) + load(k % occ)) * (rows(is, ns) + 12);
+        const double t = ((k / occ) * load(occ) + load(k % occ)) * (rows(is, ns) + 4);
         if (!IS || t < best) { best = t; IS = is; nseg = ns; }
     }
     return true;

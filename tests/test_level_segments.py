@@ -1,5 +1,6 @@
 """The cut of a one-pass matrix-core level's walk along the pulses (host code, no GPU). A segment re-reads the filter's rows,
-as far as they lie on the axis, so a cut that leaves some segment all of them costs blocks and saves nothing."""
+as far as they lie on the axis, so a cut that leaves some segment all of them costs blocks and saves nothing; and blocks
+that do not fit on a CU beside each other take turns."""
 import ctypes
 import os
 
@@ -39,3 +40,13 @@ def test_cuts_shorten_the_walk(K, pass_frac, D, monkeypatch):
                 assert n == 1 or _longest_walk(P, fp, D, n) < P, (P, C, Np, n)
                 if Np * -(-C // 8) <= 16 and P >= 400:          # few blocks, many rows: cut
                     assert n > 4, (P, C, Np, n)
+
+
+# rows of 66 and 116 outputs, blocks of five and eight waves; 12 accumulators a filter take 145 registers a thread, so
+# that a SIMD holds three waves and a CU one such block: 256 blocks fill the device
+@pytest.mark.parametrize('K,Np,C', [(108, 256, 4), (208, 256, 8), (108, 128, 9)])
+def test_blocks_that_take_turns(K, Np, C, monkeypatch):
+    monkeypatch.delenv('FSH_LMFMA_BLOCKS', raising=False)
+    fk, fp = pl.decimator_fir(K, 2, 0.6)[0], pl.decimator_fir(100, 2, 0.6)[0]
+    assert -(-fp['L'] // 2) == 12 and fk['n_out'] in (66, 116)
+    assert _segments(Np, 100, C, fk, 2, fp, 2) == 1
