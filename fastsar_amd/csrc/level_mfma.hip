@@ -502,6 +502,11 @@ bool level_mfma_shape(int Np, int P, int C, int Lk, int Dk, int Ko, int Lp, int 
         const double t = ((k / occ) * load(occ) + load(k % occ)) * (rows(is, ns) + 4);
         if (!IS || t < best) { best = t; IS = is; nseg = ns; }
     }
+    if (const char* e = getenv("FSH_LMFMA_BLOCKS")) {      // sweeps: doubled up to that many blocks
+        for (nseg = 1; nseg < Po && blocks0 * nseg < atol(e);) nseg *= 2;
+        IS = (Po + nseg - 1) / nseg;
+        nseg = (Po + IS - 1) / IS;
+    }
     return true;
 }
 

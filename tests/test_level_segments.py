@@ -50,3 +50,10 @@ def test_blocks_that_take_turns(K, Np, C, monkeypatch):
     fk, fp = pl.decimator_fir(K, 2, 0.6)[0], pl.decimator_fir(100, 2, 0.6)[0]
     assert -(-fp['L'] // 2) == 12 and fk['n_out'] in (66, 116)
     assert _segments(Np, 100, C, fk, 2, fp, 2) == 1
+
+
+def test_forced_block_count(monkeypatch):
+    fk, fp = pl.decimator_fir(108, 2, 0.6)[0], pl.decimator_fir(400, 2, 0.6)[0]
+    for blocks, want in (('1', 1), ('64', 1), ('256', 4), ('1000', 16)):
+        monkeypatch.setenv('FSH_LMFMA_BLOCKS', blocks)
+        assert _segments(64, 400, 4, fk, 2, fp, 2) == want
