@@ -10,7 +10,10 @@ namespace fsh {
 constexpr int DMAX = 4;                        // the largest decimation factor of the fused form, on either axis
 
 // Taps (uniform values) are moved to vector registers where a filter's fit VTAPS of them: a float32 fma whose operands
-// are all VGPRs issues in about 2.5 cycles a wave, one with a scalar operand in 4.4 (both at two or more waves a SIMD)
+// are all VGPRs issues in about 2.5 cycles a wave, one with a scalar operand in 4.4 (both at two or more waves a SIMD). Not
+// where the form with its factors read at run time, which keeps room for DMAX phases, would pass the 128 registers of four
+// waves a SIMD: with the rows' addresses kept for every period of its unrolled loop as well it took 140 to 211, and levels
+// that fill the device ran up to 1.8 times as long as with 70 to 112 (4,000 parents of 4 x 30 columns, 2 x 1, 85 -> 152 us)
 constexpr int VTAPS = 32;
 __device__ __forceinline__ void in_vgpr(float& v) { asm volatile("" : "+v"(v)); }
 
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
                     #pragma unroll
                     for (int s = 0; s < NWK; ++s) {
                         hk[ph][s] = (DK || ph < Dk) ? hk_t[ph * NWK + s] : 0.f;
-                        if (DL * NWK <= VTAPS) in_vgpr(hk[ph][s]);
+                        if (DL * NWK <= VTAPS && (DK || NWK + NWP <= 18)) in_vgpr(hk[ph][s]);
                     }
                 }
                 const double a = (double)ra0, b = (double)rb0;
@@ -152,7 +155,9 @@ __global__ __launch_bounds__(256) void k_level_fused(const float2* __restrict__ 
                         constexpr int q = decltype(qc)::value;
                         const int m = m0 + q;
                         if (m < mend) {
-                            const int kb = (DK ? DK : Dk) * m - plk;
+                            int kb = (DK ? DK : Dk) * m - plk;
+                            // opaque, so that the run-time form keeps no address a period and phase in registers (VTAPS)
+                            if (!DK) asm volatile("" : "+s"(kb));
                             if (kb + (DK ? DK : Dk) > 0 && kb < K) {  // a period with samples in [0, K)
                                 float2 v[DL];
                                 #pragma unroll
