@@ -82,6 +82,10 @@ bool level_fused_shape(int C, int P, int K, int Lk, int Dk, int Ko, int Lp, int 
     R = (int)std::min<size_t>(budget / per_row, (size_t)(256 / CB));
     if (R < 16 && R < P && !getenv("FSH_FUSED_LDS_KB")) R = (int)std::min<size_t>(78 * 1024 / per_row, (size_t)(256 / CB));
     R = std::min(R, P);
+    // the last rows of an axis in the chunk where 40 KB, still four blocks a CU, holds them: 800 parents of 4 x 30 columns, 30
+    // rows (29 in 39 KB) 35 -> 25 us
+    const int R40 = std::min(P, (int)std::min<size_t>(40 * 1024 / per_row, (size_t)(256 / CB)));
+    if (R >= 16 && R < P && (P + R40 - 1) / R40 < (P + R - 1) / R && !getenv("FSH_FUSED_LDS_KB")) R = R40;
     if (R < 8 && R < P) {
         // the rows' zeros do not turn a level away that fits without them
         R = std::min(P, (int)std::min<size_t>(78 * 1024 / (8 * ((size_t)(K | 1) + (size_t)CB * KoS)), (size_t)(256 / CB)));
@@ -138,7 +142,9 @@ int launch_level_fused(const float2* x, int Np, int P, int K, const float* c0, c
         const size_t per_row = 8 * ((size_t)fused_row(K, Dk) + (size_t)CB * (Ko | 1)), kb = 156 / ((G + 255) / 256);
         const int r = std::min(P, (int)std::min<size_t>(kb * 1024 / per_row, (size_t)(256 / CB)));
         if (r >= 8 || r == P) {
-            R = r;
+            // (a last chunk of a few rows shared out: 4 parents of 9 x 24 columns, 30 rows, 28 and 2 a chunk 22 -> 19 us)
+            const int chunks = (P + r - 1) / r, last = P - (chunks - 1) * r;
+            R = 4 * last <= r ? (P + chunks - 1) / chunks : r;
             lds = per_row * R;
         }
     }
