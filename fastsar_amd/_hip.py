@@ -70,6 +70,7 @@ def lib():
                             c_int, c_double, vp, vp], c_int),
         'fsh_level_mfma_noalloc': ([vp, c_int, c_int, c_int, vp, vp, c_int, vp, c_int, c_int, c_int, c_int, vp, c_int, c_int,
                                     c_int, c_int, c_double, vp, vp], c_int),
+        'fsh_fir_p_segments': ([c_int] * 3 + [P_i32], c_int),
         'fsh_level_mfma_segments': ([c_int] * 10 + [P_i32], c_int),
         'fsh_device_phases': ([vp, vp, vp, vp, c_int, c_int, c_int, c_double, c_double, vp, vp, vp], c_int),
         'fsh_final_geom': ([vp, vp, vp, c_int, c_int, P_f64, P_f64, vp, vp, vp, vp], c_int),

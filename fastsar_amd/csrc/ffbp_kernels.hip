@@ -1239,17 +1239,33 @@ bool fir_p_streams(int L, int D)
     return D >= 1 && (L + D - 1) / D <= 16 && !force;
 }
 
+// columns per thread of the streaming kernels: 2 where the launch has columns to spare (from 2^17: the 12288 x 8192 image's
+// level 1, 44.6 -> 43.5 ms), else 1 (a 512 x 512 image's first pulse filter ran 0.14 ms on one, 0.17 on two)
+static int fir_p_columns(int B, int Ko)
+{
+    const char* e = getenv("FSH_FIRP_COLS");
+    return e ? atoi(e) : ((long)B * Ko >= (1L << 17) ? 2 : 1);
+}
+
 // output pulses per segment of the streaming kernels (a thread runs down a column's rows of one segment, and the
 // segments of a column re-read ceil(L / D) - 1 periods of rows, from cache): at most 128, fewer where the columns alone
-// leave the launch short of 1,280 blocks (five a CU), not below 8. Measured, 128 against the rule: 64 x 157 columns of
-// 512 rows (62 MB) 141 -> 33 us, 48 x 301 of 1,403 186 -> 59, 64 x 264 of 3,000 380 -> 172, 64 x 352 of 4,096 425 -> 285;
-// 56 x 523 of 8,190 takes 128 either way (691 us; 745 at 24)
-static int fir_p_segment(long columns, int Po)
+// leave the launch short, not below 8. One column a thread: 1,280 blocks (five a CU). Measured, 128 against the rule: 64 x
+// 157 columns of 512 rows (62 MB) 141 -> 33 us, 48 x 301 of 1,403 186 -> 59, 64 x 264 of 3,000 380 -> 172, 64 x 352 of 4,096
+// 425 -> 285; 56 x 523 of 8,190 takes 128 either way (691 us; 745 at 24). Two columns a thread: the device holds 1,024
+// blocks, and a few past a round cost one: 400 x 352 columns of 200 rows (275 blocks a segment) 135 -> 82 us in three segments,
+// 92 in four; 1,681 x 157 of 800 rows (516) 537 us in segments of 128, 685 in two equal ones
+static int fir_p_segment(long blocks, bool two, int Po)
 {
     if (const char* e = getenv("FSH_FIRP_IC")) return std::min(Po, std::max(1, atoi(e)));          // sweeps
-    const long per = (columns + 255) / 256;
-    const int segs = (int)((1280 + per - 1) / per);
+    const int segs = (int)(two ? std::max(1L, 1024 / blocks) : (1280 + blocks - 1) / blocks);
     return std::min(Po, std::min(128, std::max(8, (Po + segs - 1) / segs)));
+}
+
+int fir_p_segments(int B, int Ko, int Po)
+{
+    const bool two = fir_p_columns(B, Ko) == 2;
+    const int IC = fir_p_segment(((long)B * (two ? (Ko + 1) / 2 : Ko) + 255) / 256, two, Po);
+    return (Po + IC - 1) / IC;
 }
 
 int launch_fir_p(const float2* y, int B, int P, int Ko, const float* taps, int L, int pl, int D, int Po, float2* z, hipStream_t s,
@@ -1273,8 +1289,6 @@ int launch_fir_p(const float2* y, int B, int P, int Ko, const float* taps, int L
     }
     const int sp = split ? 1 : 0;
     if (NW <= 16 && !(force && strcmp(force, "lds") == 0)) {
-        const int IC = fir_p_segment((long)B * Ko, Po);
-        dim3 grid((unsigned)(((long)B * Ko + 255) / 256), (Po + IC - 1) / IC);
         const bool batch = force && strcmp(force, "stream4") == 0;
         const float* rc0 = rot ? rot->c0 : nullptr;
         const float* rsl = rot ? rot->sl : nullptr;
@@ -1282,14 +1296,13 @@ int launch_fir_p(const float2* y, int B, int P, int Ko, const float* taps, int L
         const double rkc = rot ? rot->kc : 0.0;
         const char* rbe = getenv("FSH_FIRP_ROWS");                      // rows whose loads go out together: 1, 4, 8 (sweeps)
         const int rows = rbe ? atoi(rbe) : 4;
-        // columns per thread: 2 where the launch has columns to spare (from 2^17: the 12288 x 8192 image's level 1,
-        // 44.6 -> 43.5 ms), else 1 (a 512 x 512 image's first pulse filter ran 0.14 ms on one, 0.17 on two)
-        const char* cle = getenv("FSH_FIRP_COLS");
-        const int cols = cle ? atoi(cle) : ((long)B * Ko >= (1L << 17) ? 2 : 1);
-        if (!batch && cols == 2) {
-            const int H = (Ys + 1) / 2;
-            dim3 grid2((unsigned)(((long)B * H + 255) / 256), (Po + IC - 1) / IC);
-#define FSH_FP2(NN) hipLaunchKernelGGL((k_fir_p_stream2<NN>), grid2, dim3(256), (size_t)16 * D * ((NN + 3) / 4), s, y, B, P, Ko, taps, L, pl, D, Po, IC, z, hs, \
+        const bool two = !batch && fir_p_columns(B, Ko) == 2;
+        const int H = (Ys + 1) / 2;
+        const long blocks = ((long)B * (two ? H : Ko) + 255) / 256;
+        const int IC = fir_p_segment(blocks, two, Po);
+        const dim3 grid((unsigned)blocks, (Po + IC - 1) / IC);
+        if (two) {
+#define FSH_FP2(NN) hipLaunchKernelGGL((k_fir_p_stream2<NN>), grid, dim3(256), (size_t)16 * D * ((NN + 3) / 4), s, y, B, P, Ko, taps, L, pl, D, Po, IC, z, hs, \
                                        rc0, rsl, rD, rpl, rkc, Ys, sp)
             switch (NW) {
                 case 1: FSH_FP2(1); break;   case 2: FSH_FP2(2); break;   case 3: FSH_FP2(3); break;   case 4: FSH_FP2(4); break;

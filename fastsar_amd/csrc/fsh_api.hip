@@ -645,6 +645,13 @@ int fsh_level_mfma_noalloc(const float* x, int Np, int P, int K, const float* c0
     return st;
 }
 
+int fsh_fir_p_segments(int B, int Ko, int Po, int* segments)
+{
+    if (!segments || B < 1 || Ko < 1 || Po < 1) { set_error("fir_p_segments: invalid shape"); return E_INVALID; }
+    *segments = fir_p_segments(B, Ko, Po);
+    return OK;
+}
+
 int fsh_level_mfma_segments(int Np, int P, int C, int Lk, int Dk, int Ko, int Lp, int Dp, int plp, int Po, int* segments)
 {
     if (!segments) { set_error("level_mfma_segments: null argument"); return E_INVALID; }

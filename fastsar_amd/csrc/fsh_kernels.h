@@ -48,6 +48,8 @@ struct DeferredRot {
 int launch_fir_p(const float2* y, int B, int P, int Ko, const float* taps, int L, int pl, int D, int Po, float2* z,
                  hipStream_t s, const float* hs = nullptr, const DeferredRot* rot = nullptr, int ys = 0, bool split = false);
 // whether launch_fir_p takes the streaming kernel for this filter (the one that applies a deferred rho)
+// the segments of output pulses a launch_fir_p that streams cuts its columns into (rows Ko apart)
+int fir_p_segments(int B, int Ko, int Po);
 bool fir_p_streams(int L, int D);
 // the rotation and both filters of a level in one pass, for short children (fused_kernels.hip); hk_t and hp_t are the
 // polyphase tables that launch_polyphase builds from the taps (h == nullptr: the unit tap of an undecimated axis)

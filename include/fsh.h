@@ -70,6 +70,10 @@ int fsh_rot_fir_k(const float* x, int Np, int P, int K, const float* c0, const f
 int fsh_fir_p(const float* y, int B, int P, int Ko, const float* taps, int L, int pl, int D, int Po, float* z,
               void* stream);
 
+/* The segments of output pulses that a streaming fsh_fir_p (at most 16 taps a phase) cuts its columns into (host only).
+ * Results do not depend on it. No counterpart in the reference: for tests and measurements. */
+int fsh_fir_p_segments(int B, int Ko, int Po, int* segments);
+
 /* One level in one pass: fsh_rot_fir_k followed by fsh_fir_p without the intermediate y, for short children
  * (Ko <= 256, D <= 4 and ceil(L / D) <= 16 on both axes; FSH_EINVAL otherwise). x [Np, P, K], c0 and sl [Np, Cn, P], taps_k [Lk]
  * (NULL when Dk == 1), taps_p [Lp] (NULL when Dp == 1), z [Np * Cn, Po, Ko]; synchronizes the stream. Replaces the pair
