@@ -1471,15 +1471,16 @@ int launch_final_tiles(const float2* data, int B, int Pf, int Qf, int T, const d
         // T 16 and 32 at 8 lanes a block or more (fewer than 16,384 8 x 8 pixel blocks): on the matrix instructions,
         // which sum a pixel's terms in another order; larger images keep one order over (p, q) (a bright
         // pixel's rounding stands out against the image's rms by the square root of its pixels)
-        if (T >= 16 && split >= 8)
+        const bool reg = force && strcmp(force, "reg") == 0;      // the register form throughout (tests compare with it)
+        if (T >= 16 && split >= 8 && !reg)
             return launch_final_tiles_mfma(data, B, Pf, Qf, T, ux, uy, tgeo, spx, spy, a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy,
                                            nx, ny, out, s, split);
-        if (T == 32)                                         // the register form's sums, bit for bit, on the matrix cores
+        if (T == 32 && !reg)                                 // the register form's sums, bit for bit, on the matrix cores
             return launch_final_tiles_order(data, B, Pf, Qf, ux, uy, tgeo, spx, spy, a0, a1, fc2, w0, gx, gyr, tile_xy, ox, oy, nx,
                                             ny, out, s, split);
         const int per = (T / std::min(T, 8)) * (T / std::min(T, 8));
         // two threads a block where the launch's lanes come to at most a wave a SIMD (65,536): beyond, whole blocks
-        const bool half = T >= 8 && (long)B * per * split <= 65536;
+        const bool half = (T == 8 || T == 16) && (long)B * per * split <= 65536;
         const long blocks = ((long)B * per * split * (half ? 2 : 1) + 255) / 256;
         const bool w = w0 != nullptr;
 #define FSH_FR(TT, WW, HH) hipLaunchKernelGGL((k_final_tiles_reg<TT, WW, HH>), dim3((unsigned)blocks), dim3(256), 0, s, data, B, Pf, Qf, ux, uy, \
@@ -1493,7 +1494,8 @@ int launch_final_tiles(const float2* data, int B, int Pf, int Qf, int T, const d
         switch (T) {
             case 4: if (w) FSH_FR(4, true, 1); else FSH_FR(4, false, 1); break;
             case 8: FSH_FR_H(8); break;
-            default: FSH_FR_H(16); break;
+            case 16: FSH_FR_H(16); break;
+            default: if (w) FSH_FR(32, true, 1); else FSH_FR(32, false, 1); break;
         }
 #undef FSH_FR_H
 #undef FSH_FR

@@ -163,7 +163,7 @@ int launch_final_tiles_mfma(const float2* data, int B, int Pf, int Qf, int T, co
                             const float* gx, const float* gyr, const int* tile_xy, int ox, int oy, int nx, int ny, float2* out,
                             hipStream_t s, int split)
 {
-    // split 8: an image of 256 to 512 tiles of 32 x 32 or more, whose 32 x 32 blocks fill the device; 16: fewer
+    // split 8: an image of 512 to 1,023 tiles of 32 x 32 (final_split), whose 32 x 32 blocks fill the device; 16: fewer
     const int FB = T == 32 && split < 16 ? 32 : 16, PC = FinalShape<16>::PC;
     // four waves, a SIMD each (5 or 7 leave the SIMDs uneven: the 768 tiles above took 712 and 642 us); eight of 16 x 16
     // blocks with the runs to share
@@ -193,7 +193,7 @@ int launch_final_tiles_mfma(const float2* data, int B, int Pf, int Qf, int T, co
 // two waves each. Final stage of 1,536 x 1,536 pixels (116 x 78 samples a tile) 3.50 -> 1.88 ms, 2,048 x 2,048 (118 x 77)
 // 5.69 -> 3.14, 3,000 x 2,500 8.9 -> 6.3, 8,192 x 8,192 59 -> 44 (101 TFLOP/s of the float32 rate's 154): faster at every
 // size, so no 32 x 32 tile takes the register form. Bound by the matrix pipe (1,120 cycles a chunk) and the tables'
-// VALU instructions (about 500) in turn. v_mfma_f32_32x32x2_f32, a sample an instruction: 1.95 ms, 44.5.
+// VALU instructions (about 500) in turn (FSH_FINAL_KERNEL=reg takes the register form, for comparison). v_mfma_f32_32x32x2_f32, a sample an instruction: 1.95 ms, 44.5.
 namespace {
 struct OrderShape {
     static constexpr int RS = 65;                            // row stride of the tables (float2): writes free of conflicts
